@@ -254,6 +254,21 @@ int validate(const vlbm_desc* d) {
     return VLBM_OK;
 }
 
+// Interpolated bounce-back weights, for a node map that has such nodes.
+int need_ibb(vlbm_ctx* h, const uint32_t* words) {
+    if (h->ibb) return VLBM_OK;
+    size_t k = 0;
+    while (k < h->n && w_scheme(words[k]) != kInterpBB) k++;
+    if (k == h->n) return VLBM_OK;
+    void* table = nullptr;
+    int rc = dalloc(h, &table, (size_t)16 * h->d.nx * h->d.ny * h->tbytes);
+    if (rc) return rc;
+    h->ibb = table;
+    return with_params(h, [&](void* pv, auto&) {
+        return check_launch(launch_ibb_table(h->tbytes, pv, table, h->stream), "wall weight kernel");
+    });
+}
+
 int build_words(const vlbm_desc& d, std::vector<uint32_t>& out) {
     const size_t n = (size_t)d.nx * d.ny * d.nz;
     if (is_duct_builder(d.builder)) {
@@ -399,6 +414,7 @@ int vlbm_create(const vlbm_desc* d, vlbm_h* out) {
         if ((rc = dalloc(h, (void**)&h->d_mask, h->n * 4))) { release(h); return rc; }
         e = hipMemcpy(h->d_mask, h->words.data(), h->n * 4, hipMemcpyHostToDevice);
         if (e != hipSuccess) { release(h); return fail(VLBM_ERR_DEVICE, "mask upload failed"); }
+        if ((rc = need_ibb(h, h->words.data()))) { release(h); return rc; }
     }
     if ((rc = dalloc(h, (void**)&h->partials, 1024 * 3 * sizeof(double)))) { release(h); return rc; }
     if ((rc = dalloc(h, (void**)&h->out3, 3 * sizeof(double)))) { release(h); return rc; }
@@ -438,6 +454,7 @@ int vlbm_set_map(vlbm_h h, const uint32_t* words) {
         int rc = dalloc(h, (void**)&h->d_mask, h->n * 4);
         if (rc) return rc;
     }
+    if (int rc = need_ibb(h, words)) return rc;
     HIP_TRY(hipMemcpyAsync(h->d_mask, words, h->n * 4, hipMemcpyHostToDevice, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
     h->words.assign(words, words + h->n);

@@ -55,6 +55,7 @@ struct vlbm_ctx {
     long long lbm_steps = 0;  // LBM steps since init / load (the IBM stage alone does not count)
     bool resumed = false;     // loaded from a checkpoint taken after at least one step
     uint32_t* d_mask = nullptr;
+    void* ibb = nullptr;      // interpolated bounce-back weights (node maps that have such nodes)
     std::vector<uint32_t> words;   // host map
     uint32_t region_word[27];
     bool mask_geom = false;
@@ -125,6 +126,7 @@ inline void fill_params(const vlbm_ctx* h, Params<T>& p) {
     // state comes from a checkpoint of a run that has had its first one
     p.first_bc = (h->lbm_steps == 1 && !h->resumed) ? 1 : 0;
     p.mask = h->d_mask;
+    p.ibb = (const T*)h->ibb;
     p.omega_state = (T*)h->omega_state;
     p.visc_turb = (T*)h->visc_turb;
     p.m_rho = (T*)h->macr[0]; p.m_ux = (T*)h->macr[1]; p.m_uy = (T*)h->macr[2];
@@ -181,6 +183,7 @@ inline void release(vlbm_ctx* h) {
     for (void* p : h->uold) if (p) (void)hipFree(p);
     if (h->omega_state) (void)hipFree(h->omega_state);
     if (h->d_mask) (void)hipFree(h->d_mask);
+    if (h->ibb) (void)hipFree(h->ibb);
     if (h->partials) (void)hipFree(h->partials);
     if (h->out3) (void)hipFree(h->out3);
     if (h->ev0) (void)hipEventDestroy(h->ev0);

@@ -85,6 +85,19 @@ int launch_fill_feq(int q, int prec, void* state, int64_t stride, uint32_t n, co
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+int launch_ibb_table(int prec, const void* params, void* table, void* stream) {
+    if (prec == 8) {
+        const Params<double>& p = *(const Params<double>*)params;
+        hipLaunchKernelGGL((k_ibb_table<double>), grid_for((uint32_t)(p.nx * p.ny)), dim3(kBlock), 0, (hipStream_t)stream, p,
+                           (double*)table);
+    } else {
+        const Params<float>& p = *(const Params<float>*)params;
+        hipLaunchKernelGGL((k_ibb_table<float>), grid_for((uint32_t)(p.nx * p.ny)), dim3(kBlock), 0, (hipStream_t)stream, p,
+                           (float*)table);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 int launch_reduce(int prec, const void* rho, const void* ux, const void* uy, const void* uz, void* ux_old,
                   void* uy_old, void* uz_old, uint32_t n, double* partials, double* out3, void* stream) {
     hipStream_t st = (hipStream_t)stream;

@@ -198,18 +198,18 @@ __device__ __forceinline__ T load_pop(const Params<T>& p, int i, uint32_t node) 
 //     (VelZouHe.cu:104-119, PresZouHe.cu:103-119).
 // Zou-He works on deviations unchanged: the weights of T + 2K sum to 1 and
 // the tangential sums are antisymmetric.
-template <typename T>
-__device__ __forceinline__ void zou_he(T* g, int dir, bool pressure, T uxw, T uyw, T uzw, T rhow_in,
-                                       bool compat) {
-    if (dir > dB) return;
-    const int a = (dir == dN || dir == dS) ? 1 : ((dir == dW || dir == dE) ? 0 : 2);
-    const int s = (dir == dN || dir == dE || dir == dF) ? 1 : -1;
+// The face is a template parameter: sums, signs and the incoming set are then
+// constants, and the face updates in place (an incoming population takes its
+// opposite, which is outgoing, or itself).
+template <int DIR, typename T>
+__device__ __forceinline__ void zou_he_face(T* g, bool pressure, T uxw, T uyw, T uzw, T rhow_in, bool compat) {
+    constexpr int a = (DIR == dN || DIR == dS) ? 1 : ((DIR == dW || DIR == dE) ? 0 : 2);
+    constexpr int s = (DIR == dN || DIR == dE || DIR == dF) ? 1 : -1;
     auto ca = [&](int i) -> int { return a == 0 ? kCX[i] : (a == 1 ? kCY[i] : kCZ[i]); };
     // the reference's EAST lines sum the WEST face's known set (c_x = -1, the
     // EAST face's incoming populations) into T + 2K (VelZouHe.cu:104-108,
     // PresZouHe.cu:103-107)
-    const int known = (compat && dir == dE) ? -s : s;
-    T tsum = 0, ksum = 0, n_t[3] = {0, 0, 0};
+    T tsum = 0, ksum = 0, kother = 0, n_t[3] = {0, 0, 0};
 #pragma unroll
     for (int i = 0; i < 19; i++) {
         const int c = ca(i);
@@ -218,10 +218,13 @@ __device__ __forceinline__ void zou_he(T* g, int dir, bool pressure, T uxw, T uy
             n_t[0] += (T)kCX[i] * g[i];
             n_t[1] += (T)kCY[i] * g[i];
             n_t[2] += (T)kCZ[i] * g[i];
-        } else if (c == known) {
+        } else if (c == s) {
             ksum += g[i];
+        } else {
+            kother += g[i];
         }
     }
+    if (DIR == dE && compat) ksum = kother;
     const T tk = tsum + 2 * ksum;     // (T + 2K) - 1 in deviations
     T u[3] = {uxw, uyw, uzw};
     T rho_w;
@@ -232,34 +235,40 @@ __device__ __forceinline__ void zou_he(T* g, int dir, bool pressure, T uxw, T uy
         u[a] = (T)s * un;
     } else {
         T denom = (T)1 + (T)s * u[a];
-        if (compat && dir == dB) denom = (T)1 + uzw;
+        if (DIR == dB && compat) denom = (T)1 + uzw;
         rho_w = ((T)1 + tk) / denom;
     }
     T nt[3];
 #pragma unroll
     for (int t = 0; t < 3; t++) nt[t] = (T)0.5 * n_t[t] - (pressure ? (T)0 : rho_w * u[t] / (T)3);
     nt[a] = 0;
-    const bool east_compat = compat && dir == dE;
-    T out[19];
-#pragma unroll
-    for (int i = 1; i < 19; i++) out[i] = g[i];
+    // increment of population j's formula
+    auto increment = [&](int j) -> T {
+        T cu = (T)kCX[j] * u[0] + (T)kCY[j] * u[1] + (T)kCZ[j] * u[2];
+        if (DIR == dB && (j == 11 || j == 18) && compat && !pressure) cu = (T)kCZ[j] * u[2] + (T)kCY[j] * u[0];
+        if ((DIR == dW || DIR == dE) && j == 15 && compat && !pressure) cu = (T)kCX[j] * u[0] + (T)kCZ[j] * u[1];
+        const T corr = (T)kCX[j] * nt[0] + (T)kCY[j] * nt[1] + (T)kCZ[j] * nt[2];
+        return (T)(6.0 * weight<19>(j)) * rho_w * cu - corr;
+    };
 #pragma unroll
     for (int i = 1; i < 19; i++) {
         if (ca(i) != -s) continue;                  // incoming populations only
-        const int j = east_compat ? opp(i) : i;     // population whose formula is used
-        T cu;
-        if (compat && !pressure && dir == dB && (j == 11 || j == 18))
-            cu = (T)kCZ[j] * u[2] + (T)kCY[j] * u[0];
-        else if (compat && !pressure && (dir == dW || dir == dE) && j == 15)
-            cu = (T)kCX[j] * u[0] + (T)kCZ[j] * u[1];
-        else
-            cu = (T)kCX[j] * u[0] + (T)kCY[j] * u[1] + (T)kCZ[j] * u[2];
-        const T corr = (T)kCX[j] * nt[0] + (T)kCY[j] * nt[1] + (T)kCZ[j] * nt[2];
-        const T inc = (T)(6.0 * weight<19>(j)) * rho_w * cu - corr;
-        out[i] = (east_compat ? g[i] : g[opp(i)]) + inc;
+        if (DIR == dE && compat) g[i] = g[i] + increment(opp(i));
+        else g[i] = g[opp(i)] + increment(i);
     }
-#pragma unroll
-    for (int i = 1; i < 19; i++) g[i] = out[i];
+}
+
+template <typename T>
+__device__ __forceinline__ void zou_he(T* g, int dir, bool pressure, T uxw, T uyw, T uzw, T rhow_in, bool compat) {
+    switch (dir) {
+    case dN: zou_he_face<dN>(g, pressure, uxw, uyw, uzw, rhow_in, compat); break;
+    case dS: zou_he_face<dS>(g, pressure, uxw, uyw, uzw, rhow_in, compat); break;
+    case dW: zou_he_face<dW>(g, pressure, uxw, uyw, uzw, rhow_in, compat); break;
+    case dE: zou_he_face<dE>(g, pressure, uxw, uyw, uzw, rhow_in, compat); break;
+    case dF: zou_he_face<dF>(g, pressure, uxw, uyw, uzw, rhow_in, compat); break;
+    case dB: zou_he_face<dB>(g, pressure, uxw, uyw, uzw, rhow_in, compat); break;
+    default: break;
+    }
 }
 
 // Velocity bounce-back (src/CUDA/boundaryConditionsSchemes/D3Q19_VelBounceBack.cu:27-149):
@@ -273,17 +282,13 @@ __device__ __forceinline__ void vel_bounce_back(T* g, int dir, T uxw, T uyw, T u
     for (int i = 0; i < Q; i++) dr += g[i];
     const T rho = (T)1 + dr;
     const unsigned faces = kDirFaces[dir];
-    T out[Q];
-#pragma unroll
-    for (int i = 0; i < Q; i++) out[i] = g[i];
+    // in place: the opposite of a single face's incoming population is outgoing
 #pragma unroll
     for (int i = 1; i < Q; i++) {
-        if (!incoming(i, faces)) continue;
         const T cu = (T)kCX[i] * uxw + (T)kCY[i] * uyw + (T)kCZ[i] * uzw;
-        out[i] = g[opp(i)] + (T)(6.0 * weight<Q>(i)) * rho * cu;
+        const T v = g[opp(i)] + (T)(6.0 * weight<Q>(i)) * rho * cu;
+        g[i] = incoming(i, faces) ? v : g[i];
     }
-#pragma unroll
-    for (int i = 0; i < Q; i++) g[i] = out[i];
 }
 
 // Interpolated bounce-back (Bouzidi, linear) against the duct circle(s)
@@ -318,54 +323,91 @@ __device__ T wall_q(int kind, T x1, T y1, T x2, T y2, T R) {
     }
 }
 
+// The interpolation weights depend on the column (x, y), the direction and the
+// wall only. Both of the reference's forms
+//   q > 1/2:  (1/2q) f_opp(x) + ((q - 1/2)/q) f_i(x) + 6 w_i c_i.u_w / 2q
+//   else:     2q f_opp(x) + (1 - 2q) f_opp(x + c_i) + 6 w_i c_i.u_w
+// are a f_opp(x) + (1 - a) far + 6 w_i c_i.u_w s with one number a per
+// direction; the table holds it, negative for q > 1/2. A step that evaluates
+// q (two square roots and five divisions) at every wall node and plane spends
+// most of its time there: a circular duct crosses nearly every 64-node row.
+constexpr int kIbbDirs = 8;
+template <typename T>
+__device__ __forceinline__ size_t ibb_index(const Params<T>& p, int x, int y, int b, bool inside) {
+    return ((size_t)(inside ? kIbbDirs + b : b) * (size_t)p.ny + (size_t)y) * (size_t)p.nx + (size_t)x;
+}
+
+// D2Q9 projections in the reference's bit order (nodeTypeMap.h:100-107)
+__host__ __device__ constexpr int ibb_dx(int b) { return (b == 0 || b == 4 || b == 7) ? 1 : ((b == 2 || b == 5 || b == 6) ? -1 : 0); }
+__host__ __device__ constexpr int ibb_dy(int b) { return (b == 1 || b == 4 || b == 5) ? 1 : ((b == 3 || b == 6 || b == 7) ? -1 : 0); }
+__host__ __device__ constexpr int ibb_kind(int b) { return b < 4 ? (b & 1) : 2 + (b & 1); }
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_ibb_table(const Params<T> p, T* table) {
+    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+    if (t >= (uint32_t)p.nx * (uint32_t)p.ny) return;
+    const int x = (int)(t % (uint32_t)p.nx), y = (int)(t / (uint32_t)p.nx);
+    const T xN = (T)x - (T)(p.nx - 1) / (T)2, yN = (T)y - (T)(p.ny - 1) / (T)2;
+    for (int wall = 0; wall < 2; wall++)
+        for (int b = 0; b < kIbbDirs; b++) {
+            const T q = wall_q<T>(ibb_kind(b), xN, yN, xN - (T)ibb_dx(b), yN - (T)ibb_dy(b), wall ? p.duct_r : p.duct_R);
+            table[ibb_index(p, x, y, b, wall != 0)] = q > (T)0.5 ? -((T)0.5 / q) : 2 * q;
+        }
+}
+
 template <int Q, typename T, class PC>
-__device__ void interp_bounce_back(T* g, const Params<T>& p, const Node<T>& nd, unsigned unknown, bool inside,
-                                   PC pc) {
-    // D2Q9 projections in the reference's bit order (nodeTypeMap.h:100-107)
-    const int dxs[8] = {1, 0, -1, 0, 1, -1, -1, 1};
-    const int dys[8] = {0, 1, 0, -1, 1, 1, -1, -1};
-    const int kinds[8] = {0, 1, 0, 1, 2, 3, 2, 3};
-    const T xN = (T)nd.x - (T)(p.nx - 1) / (T)2, yN = (T)nd.y - (T)(p.ny - 1) / (T)2;
-    const T rr = sqrt(xN * xN + yN * yN);
-    const T c = xN / rr, s = yN / rr;
-    T radius, uxw, uyw, uzw;
-    if (inside) {
-        radius = p.duct_r; uxw = -p.w_in * radius * s; uyw = p.w_in * radius * c; uzw = p.u_in;
-    } else {
-        const T wo = p.w_out * ((T)nd.z / (T)p.nz);
-        radius = p.duct_R; uxw = -wo * radius * s; uyw = wo * radius * c; uzw = p.u_out;
+__device__ __forceinline__ void interp_bounce_back(T* g, const Params<T>& p, const Node<T>& nd, unsigned unknown,
+                                                   bool inside, PC pc) {
+    T uxw = 0, uyw = 0, uzw = inside ? p.u_in : p.u_out;
+    const T turn = inside ? p.w_in : p.w_out;
+    if (turn != (T)0) {
+        const T xN = (T)nd.x - (T)(p.nx - 1) / (T)2, yN = (T)nd.y - (T)(p.ny - 1) / (T)2;
+        const T rr = sqrt(xN * xN + yN * yN);
+        const T wr = inside ? turn * p.duct_r : turn * ((T)nd.z / (T)p.nz) * p.duct_R;
+        uxw = -wr * (yN / rr);
+        uyw = wr * (xN / rr);
     }
-    for (int b = 0; b < 8; b++) {
-        if (!(unknown & (1u << b))) continue;
-        const T qd = wall_q<T>(kinds[b], xN, yN, xN - (T)dxs[b], yN - (T)dys[b], radius);
+    pc.walls(inside);
+    // New value of population i from the post-collision fi, fj = f_opp of the
+    // node and the opposite population at x + c_i, which the gather brought to
+    // x. (The reference reads x + c_i unwrapped; the gather wraps, which keeps
+    // degenerate, 1-2 node wide lattices in bounds and is the same node otherwise.)
+    auto from_wall = [&](int i, T a, T fi, T fj, T at_opp) -> T {
+        const T cu = (T)kCX[i] * uxw + (T)kCY[i] * uyw + (T)kCZ[i] * uzw;
+        T fa = at_opp;
+        // rheometer: the reference refills an unused plane's populations
+        // toward the plates from its extra z plane (the rest state) in
+        // every step's stream, so only the first boundary pass sees the
+        // initial values there
+        if (PC::kPlates && p.plates) {
+            const int za = (int)nd.z + kCZ[i];
+            if (za == 0 || za == p.nz - 1) fa = p.first_bc ? pc.memory(opp(i), kCX[i], kCY[i], kCZ[i]) : (T)0;
+        }
+        const bool node = a < (T)0;
+        const T m = fabs(a);
+        return m * fj + ((T)1 - m) * (node ? fi : fa) + (T)(6.0 * weight<Q>(i)) * cu * (node ? m : (T)1);
+    };
+    // line by line of the projection: b and b + 2 are opposite, and both can
+    // be unknown, so a pair takes its streamed values before either is set
 #pragma unroll
-        for (int i = 1; i < Q; i++) {
-            if (kCX[i] != dxs[b] || kCY[i] != dys[b]) continue;
-            const int j = opp(i);
-            const T cu = (T)kCX[i] * uxw + (T)kCY[i] * uyw + (T)kCZ[i] * uzw;
-            const T df = (T)weight<Q>(i) * cu;
-            const T fj = pc(j, 0, 0, 0);
-            if (qd > (T)0.5) {
-                const T fi = pc(i, 0, 0, 0);
-                g[i] = ((T)0.5 / qd) * fj + ((qd - (T)0.5) / qd) * fi + (T)3 * df / qd;
-            } else {
-                // the reference reads x + c_i unwrapped; wrapping keeps degenerate
-                // (1-2 node wide) lattices in bounds and is the same node otherwise
-                T fa = pc(j, kCX[i], kCY[i], kCZ[i]);
-                // rheometer: the reference refills an unused plane's populations
-                // toward the plates from its extra z plane (the rest state) in
-                // every step's stream, so only the first boundary pass sees the
-                // initial values there
-                if (p.plates && !p.first_bc) {
-                    const int za = (int)nd.z + kCZ[i];
-                    if (za == 0 || za == p.nz - 1) fa = (T)0;
-                }
-                g[i] = 2 * qd * fj + (1 - 2 * qd) * fa + (T)6 * df;
+    for (int b = 0; b < 6; b++) {
+        if (b == 2 || b == 3) continue;
+        const bool fwd = unknown & (1u << b), bwd = unknown & (4u << b);
+        if (fwd || bwd) {
+            const T af = pc.wall(b, inside), ab = pc.wall(b + 2, inside);
+#pragma unroll
+            for (int i = 1; i < Q; i++) {
+                if (kCX[i] != ibb_dx(b) || kCY[i] != ibb_dy(b)) continue;
+                const int j = opp(i);
+                pc.fence();
+                const T fi = pc(i, 0, 0, 0), fj = pc(j, 0, 0, 0);
+                const T vi = from_wall(i, af, fi, fj, g[j]), vj = from_wall(j, ab, fj, fi, g[i]);
+                g[i] = fwd ? vi : g[i];
+                g[j] = bwd ? vj : g[j];
             }
         }
     }
 }
-
 
 // ---------------------------------------------------------------------------
 // Per-node pieces
@@ -402,18 +444,63 @@ __device__ __forceinline__ uint32_t node_word(const Params<T>& p, const Node<T>&
 // c_i, so the coefficients hold the post-collision populations exactly.
 // ---------------------------------------------------------------------------
 
-// g*_i of the node from its 10 coefficients at c (element stride st).
+// Post-collision populations of 10 coefficients. Opposite pairs share the
+// even part E = A + c^T G c and the odd part O = B.c: g = w E +- w O. Each
+// sum has one fixed association and the products are explicit fused
+// multiply-adds, so a population has the same bits wherever it is expanded.
+template <int Q, typename T>
+__device__ __forceinline__ void expand(const T* c, T* g) {
+    const T A = c[0], bx = c[1], by = c[2], bz = c[3];
+    const T w1 = (T)weight<Q>(1), w2 = (T)weight<Q>(7);
+    const T ex = A + c[4], ey = A + c[5], ez = A + c[6];
+    const T exy = ex + c[5], exz = ex + c[6], eyz = ey + c[6];
+    auto pair = [&](int i, T w, T even, T odd) {
+        const T t = w * even;
+        g[i] = fma(w, odd, t);
+        g[i + 1] = fma(-w, odd, t);
+    };
+    g[0] = (T)weight<Q>(0) * A;
+    pair(1, w1, ex, bx);
+    pair(3, w1, ey, by);
+    pair(5, w1, ez, bz);
+    pair(7, w2, exy + c[7], bx + by);
+    pair(9, w2, exz + c[8], bx + bz);
+    pair(11, w2, eyz + c[9], by + bz);
+    pair(13, w2, exy - c[7], bx - by);
+    pair(15, w2, exz - c[8], bx - bz);
+    pair(17, w2, eyz - c[9], by - bz);
+    if constexpr (Q == 27) {
+        const T w3 = (T)weight<27>(19);
+        const T e = exy + c[6];
+        const T p = e + c[7], m = e - c[7], sp = c[8] + c[9], sm = c[8] - c[9];
+        const T op = bx + by, om = bx - by;
+        pair(19, w3, p + sp, op + bz);        // ( 1,  1,  1)
+        pair(21, w3, p - sp, op - bz);        // ( 1,  1, -1)
+        pair(23, w3, m + sm, om + bz);        // ( 1, -1,  1)
+        pair(25, w3, m - sm, bz - om);        // (-1,  1,  1)
+    }
+}
+
+// g*_i of the node from its 10 coefficients at c (element stride st), with
+// the sums and products of expand(), so both give the same bits.
 template <int Q, typename T, typename P>
 __device__ __forceinline__ T recon(int i, const P* c, int64_t st) {
     const int cx = kCX[i], cy = kCY[i], cz = kCZ[i];
-    T v = (T)c[0];
-    if (cx) v += (T)cx * (T)c[1 * st] + (T)c[4 * st];
-    if (cy) v += (T)cy * (T)c[2 * st] + (T)c[5 * st];
-    if (cz) v += (T)cz * (T)c[3 * st] + (T)c[6 * st];
-    if (cx * cy) v += (T)(cx * cy) * (T)c[7 * st];
-    if (cx * cz) v += (T)(cx * cz) * (T)c[8 * st];
-    if (cy * cz) v += (T)(cy * cz) * (T)c[9 * st];
-    return (T)weight<Q>(i) * v;
+    const T w = (T)weight<Q>(i);
+    T e = (T)c[0];
+    if (cx) e += (T)c[4 * st];
+    if (cy) e += (T)c[5 * st];
+    if (cz) e += (T)c[6 * st];
+    if (cx * cy) e += (T)(cx * cy) * (T)c[7 * st];
+    if (cx * cy * cz) e += (T)(cx * cz) * (T)c[8 * st] + (T)(cy * cz) * (T)c[9 * st];
+    else if (cx * cz) e += (T)(cx * cz) * (T)c[8 * st];
+    else if (cy * cz) e += (T)(cy * cz) * (T)c[9 * st];
+    if (i == 0) return w * e;
+    T o = 0;
+    if (cx) o = (T)cx * (T)c[1 * st];
+    if (cy) o = cx ? o + (T)cy * (T)c[2 * st] : (T)cy * (T)c[2 * st];
+    if (cz) o = cx || cy ? o + (T)cz * (T)c[3 * st] : (T)cz * (T)c[3 * st];
+    return fma(w, o, w * e);
 }
 
 // Node at offset (dx, dy, dz) in {-1, 0, 1}^3 from nd, wrapped.
@@ -436,9 +523,15 @@ struct GlobalPC {
         if (IN == kRepPop) return load_pop<S, T>(p, i, node);
         return recon<Q, T, S>(i, (const S*)p.src + node, p.stride);
     }
+    __device__ __forceinline__ T memory(int i, int dx, int dy, int dz) const { return (*this)(i, dx, dy, dz); }
     // coefficient states: the node's own 10 coefficients, read once for the
     // several populations a bounce-back rebuilds from them
     static constexpr bool kCoefs = IN == kRepMom;
+    static constexpr bool kPlates = IN == kRepPop;      // the rheometer is refused for coefficients
+    __device__ __forceinline__ void fence() const {}
+    // wall weights of the column (ibb_index)
+    __device__ __forceinline__ void walls(bool) const {}
+    __device__ __forceinline__ T wall(int b, bool inside) const { return p.ibb[ibb_index(p, nd.x, nd.y, b, inside)]; }
     __device__ __forceinline__ void own(T* c) const {
 #pragma unroll
         for (int k = 0; k < kCoef; k++) c[k] = (T)((const S*)p.src)[(int64_t)k * p.stride + nd.idx];
@@ -579,6 +672,34 @@ __device__ __forceinline__ void plate_held(T* g, const Params<T>& p, const Node<
     }
 }
 
+// Specular reflection on a face: incoming i comes from the mirror population
+// of the node displaced by minus the tangential part of c_i
+// (src/CUDA/boundaryConditionsSchemes/freeSlip.cu:26-168).
+template <int Q, int DIR, typename T, class PC>
+__device__ __forceinline__ void free_slip_face(T* g, PC pc) {
+    constexpr bool fx = DIR == dW || DIR == dE, fy = DIR == dN || DIR == dS, fz = DIR == dF || DIR == dB;
+#pragma unroll
+    for (int i = 1; i < Q; i++) {
+        if (!incoming(i, kDirFaces[DIR])) continue;
+        const int cx = kCX[i], cy = kCY[i], cz = kCZ[i];
+        g[i] = pc.memory(find_pop(fx ? -cx : cx, fy ? -cy : cy, fz ? -cz : cz), fx ? 0 : -cx, fy ? 0 : -cy, fz ? 0 : -cz);
+    }
+}
+
+// Halfway bounce-back from the node's 10 coefficients: the populations of mask
+// m take their opposites' post-collision values, with the sums and products of
+// expand(). Pair by pair, so no more than two of them are live at once.
+template <int Q, typename T>
+__device__ __forceinline__ void bounce_back(T* g, const T* c, uint32_t m) {
+#pragma unroll
+    for (int i = 1; i < Q; i += 2) {
+        const T v = recon<Q, T, T>(i, c, 1), w = recon<Q, T, T>(i + 1, c, 1);
+        g[i] = m & (1u << i) ? w : g[i];
+        g[i + 1] = m & (2u << i) ? v : g[i + 1];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // Boundary condition of the node's word on the gathered populations
 // (dispatch of src/CUDA/boundaryConditionsHandler.cu:25-79); pc gives the
 // post-collision populations of the node and its neighbours. MASK: the words
@@ -590,48 +711,31 @@ __device__ __forceinline__ void apply_bc(T* g, const Params<T>& p, const Node<T>
     const int scheme = w_scheme(word);
     const int dir = w_dir(word);
     if constexpr (MASK) {
-        if (p.plates) plate_held<Q, T>(g, p, nd, pc);
+        if (PC::kPlates && p.plates) plate_held<Q, T>(g, p, nd, pc);
     }
     if (scheme == kBounceBack) {
         // convex edges/corners carry no bounce-back (boundaryConditionsHandler.cu:158-256)
         if (dir >= dNW && w_geom(word)) return;
         if (dir > dSEB) return;
         const uint32_t m = (Q == 19) ? c_bb19.m[dir] : c_bb27.m[dir];
-        if constexpr (PC::kCoefs && Q == 19) {
+        if constexpr (PC::kCoefs) {
             T c[kCoef];
             pc.own(c);
-#pragma unroll
-            for (int i = 1; i < Q; i++)
-                if (m & (1u << i)) g[i] = recon<Q, T, T>(opp(i), c, 1);
+            bounce_back<Q, T>(g, c, m);
         } else {
 #pragma unroll
             for (int i = 1; i < Q; i++)
                 if (m & (1u << i)) g[i] = pc(opp(i), 0, 0, 0);
         }
     } else if (scheme == kFreeSlip) {
-        // specular reflection: incoming i comes from the mirror population m
-        // of the node displaced by minus the tangential part of c_i
-        // (src/CUDA/boundaryConditionsSchemes/freeSlip.cu:26-168)
-        if (dir > dB) return;
-        const unsigned faces = kDirFaces[dir];
-#pragma unroll
-        for (int i = 1; i < Q; i++) {
-            if (!incoming(i, faces)) continue;
-            // the source node is displaced by minus the tangential part of c_i
-            int mx = kCX[i], my = kCY[i], mz = kCZ[i];
-            int ox = -mx, oy = -my, oz = -mz;
-            if (dir == dN || dir == dS) {
-                my = -my;
-                oy = 0;
-            } else if (dir == dW || dir == dE) {
-                mx = -mx;
-                ox = 0;
-            } else {
-                mz = -mz;
-                oz = 0;
-            }
-            const int m = find_pop(mx, my, mz);
-            g[i] = pc(m, ox, oy, oz);
+        switch (dir) {
+        case dN: free_slip_face<Q, dN>(g, pc); break;
+        case dS: free_slip_face<Q, dS>(g, pc); break;
+        case dW: free_slip_face<Q, dW>(g, pc); break;
+        case dE: free_slip_face<Q, dE>(g, pc); break;
+        case dF: free_slip_face<Q, dF>(g, pc); break;
+        case dB: free_slip_face<Q, dB>(g, pc); break;
+        default: break;
         }
     } else if (scheme == kVelBB) {
         if (Q == 19)
@@ -643,7 +747,7 @@ __device__ __forceinline__ void apply_bc(T* g, const Params<T>& p, const Node<T>
     } else if constexpr (MASK) {
         if (scheme == kInterpBB) {
             interp_bounce_back<Q, T>(g, p, nd, w_interp(word), dir == dS, pc);
-        } else if (scheme == kSpecial) {
+        } else if (PC::kPlates && scheme == kSpecial) {
             if (Q == 19 && (dir == dF || dir == dB)) rheometer_plate<Q, T>(g, p, nd, dir == dF);
         }
     }
@@ -672,22 +776,43 @@ __device__ __forceinline__ uint32_t tile_of(const Params<T>& p, int x, int y, in
     return tile_index(x, y, z, p.tiles_x, p.tiles_y);
 }
 
+// 16-bit storage keeps the sums and products of the collision in one order:
+// stochastic rounding turns a change in the last bit of a float into a whole
+// step of the stored 16-bit value.
+template <typename S> constexpr bool kSequential = sizeof(S) == 2;
+
 // omega_old: power-law state of the node (ignored otherwise).
-template <int Q, int RHEO, typename T>
+template <int Q, int RHEO, bool SEQ, typename T>
 __device__ __forceinline__ Moments<Q, RHEO, T> moments(const T* g, const Params<T>& p, T omega_old,
                                                        const Force<T>& F) {
     Moments<Q, RHEO, T> m;
-    T dr = 0, jx = 0, jy = 0, jz = 0, sxx = 0, syy = 0, szz = 0, sxy = 0, sxz = 0, syz = 0;
+    T dr = SEQ ? (T)0 : g[0], jx = 0, jy = 0, jz = 0, sxx = 0, syy = 0, szz = 0, sxy = 0, sxz = 0, syz = 0;
+    if constexpr (SEQ) {
 #pragma unroll
-    for (int i = 0; i < Q; i++) {
-        const T v = g[i];
-        dr += v;
-        if (kCX[i]) { jx += (T)kCX[i] * v; sxx += v; }
-        if (kCY[i]) { jy += (T)kCY[i] * v; syy += v; }
-        if (kCZ[i]) { jz += (T)kCZ[i] * v; szz += v; }
-        if (kCX[i] * kCY[i]) sxy += (T)(kCX[i] * kCY[i]) * v;
-        if (kCX[i] * kCZ[i]) sxz += (T)(kCX[i] * kCZ[i]) * v;
-        if (kCY[i] * kCZ[i]) syz += (T)(kCY[i] * kCZ[i]) * v;
+        for (int i = 0; i < Q; i++) {
+            const T v = g[i];
+            dr += v;
+            if (kCX[i]) { jx += (T)kCX[i] * v; sxx += v; }
+            if (kCY[i]) { jy += (T)kCY[i] * v; syy += v; }
+            if (kCZ[i]) { jz += (T)kCZ[i] * v; szz += v; }
+            if (kCX[i] * kCY[i]) sxy += (T)(kCX[i] * kCY[i]) * v;
+            if (kCX[i] * kCZ[i]) sxz += (T)(kCX[i] * kCZ[i]) * v;
+            if (kCY[i] * kCZ[i]) syz += (T)(kCY[i] * kCZ[i]) * v;
+        }
+    } else {
+        // over the opposite pairs (i, i + 1): the even moments take g_i +
+        // g_(i+1), the first moments g_i - g_(i+1), half the additions
+#pragma unroll
+        for (int i = 1; i < Q; i += 2) {
+            const T s = g[i] + g[i + 1], d = g[i] - g[i + 1];
+            dr += s;
+            if (kCX[i]) { jx += (T)kCX[i] * d; sxx += s; }
+            if (kCY[i]) { jy += (T)kCY[i] * d; syy += s; }
+            if (kCZ[i]) { jz += (T)kCZ[i] * d; szz += s; }
+            if (kCX[i] * kCY[i]) sxy += (T)(kCX[i] * kCY[i]) * s;
+            if (kCX[i] * kCZ[i]) sxz += (T)(kCX[i] * kCZ[i]) * s;
+            if (kCY[i] * kCZ[i]) syz += (T)(kCY[i] * kCZ[i]) * s;
+        }
     }
     const T rho = (T)1 + dr;
     const T inv = (T)1 / rho;
@@ -695,7 +820,7 @@ __device__ __forceinline__ Moments<Q, RHEO, T> moments(const T* g, const Params<
     const T uy = (jy + (T)0.5 * F.y) * inv;
     const T uz = (jz + (T)0.5 * F.z) * inv;
     // Pi^neq = sum f c c - rho (u u + I/3) = sum g c c - rho u u - (rho-1)/3 I
-    const T dr3 = dr / (T)3;
+    const T dr3 = SEQ ? dr / (T)3 : dr * (T)(1.0 / 3);
     m.pxx = sxx - rho * ux * ux - dr3;
     m.pyy = syy - rho * uy * uy - dr3;
     m.pzz = szz - rho * uz * uz - dr3;
@@ -744,13 +869,50 @@ __device__ __forceinline__ Moments<Q, RHEO, T> moments(const T* g, const Params<
     return m;
 }
 
-// Regularized collision with Guo forcing, in deviation form:
+// Regularized collision with Guo forcing (src/CUDA/lbm.cu:263-461), in
+// deviation form
 //   g*_i = w_i [ (rho-1) + rho (3 c.u + 4.5 (c.u)^2 - 1.5 u.u) ]
 //        + (1-omega) 4.5 w_i (Q_i : Pi^neq - c_i.F/3)
-//        + (1-omega/2) w_i (3 c.F + 9 (c.u)(c.F) - 3 u.F)
-// with Q_i = c_i c_i - I/3 (src/CUDA/lbm.cu:263-461).
+//        + (1-omega/2) w_i (3 c.F + 9 (c.u)(c.F) - 3 u.F),  Q_i = c_i c_i - I/3,
+// as the coefficients of w_i (A + B.c + c^T G c):
+//   A    = (rho-1) - 1.5 rho u.u - a tr(Pi)/3 - 3 b u.F
+//   B_a  = 3 rho u_a + (3 b - a/3) F_a
+//   G_aa = 4.5 rho u_a^2 + 9 b u_a F_a + a Pi_aa
+//   G_ab = 9 rho u_a u_b + 9 b (u_a F_b + u_b F_a) + 2 a Pi_ab      (a < b)
+// with a = 4.5 (1 - omega), b = 1 - omega/2.
+template <int Q, int RHEO, typename T>
+__device__ __forceinline__ void coeffs_collide(T* c, const Moments<Q, RHEO, T>& m, const Force<T>& F) {
+    const T om = m.omega;
+    const T a = (T)4.5 * ((T)1 - om);
+    const T b = (T)1 - (T)0.5 * om;
+    const T uf = m.ux * F.x + m.uy * F.y + m.uz * F.z;
+    const T usq = m.ux * m.ux + m.uy * m.uy + m.uz * m.uz;
+    const T tr = m.pxx + m.pyy + m.pzz;
+    const T r3 = (T)3 * m.rho, r45 = (T)4.5 * m.rho, r9 = (T)9 * m.rho;
+    const T bf = (T)3 * b - (T)1.5 * ((T)1 - om), b9 = (T)9 * b, a2 = (T)2 * a;
+    c[0] = m.dr - (T)1.5 * m.rho * usq - (T)1.5 * ((T)1 - om) * tr - (T)3 * b * uf;
+    c[1] = r3 * m.ux + bf * F.x;
+    c[2] = r3 * m.uy + bf * F.y;
+    c[3] = r3 * m.uz + bf * F.z;
+    c[4] = r45 * m.ux * m.ux + b9 * m.ux * F.x + a * m.pxx;
+    c[5] = r45 * m.uy * m.uy + b9 * m.uy * F.y + a * m.pyy;
+    c[6] = r45 * m.uz * m.uz + b9 * m.uz * F.z + a * m.pzz;
+    c[7] = r9 * m.ux * m.uy + b9 * (m.ux * F.y + m.uy * F.x) + a2 * m.pxy;
+    c[8] = r9 * m.ux * m.uz + b9 * (m.ux * F.z + m.uz * F.x) + a2 * m.pxz;
+    c[9] = r9 * m.uy * m.uz + b9 * (m.uy * F.z + m.uz * F.y) + a2 * m.pyz;
+}
+
+// The regularized collision as populations.
 template <int Q, int RHEO, typename T>
 __device__ __forceinline__ void collide(T* g, const Moments<Q, RHEO, T>& m, const Force<T>& F) {
+    T c[kCoef];
+    coeffs_collide<Q, RHEO, T>(c, m, F);
+    expand<Q, T>(c, g);
+}
+
+// The same collision population by population (kSequential).
+template <int Q, int RHEO, typename T>
+__device__ __forceinline__ void collide_seq(T* g, const Moments<Q, RHEO, T>& m, const Force<T>& F) {
     const T om = m.omega;
     const T a = (T)4.5 * ((T)1 - om);
     const T b = (T)1 - (T)0.5 * om;
@@ -804,51 +966,29 @@ __device__ __forceinline__ void collide_bgk(T* g, const Moments<Q, RHEO, T>& m, 
     }
 }
 
-// Regularized collision in coefficient form (kRepMom): the same g*_i as
-// collide(), as A + B.c + c^T G c with
-//   A    = (rho-1) - 1.5 rho u.u - a tr(Pi)/3 - 3 b u.F
-//   B_a  = 3 rho u_a + (3 b - a/3) F_a
-//   G_aa = 4.5 rho u_a^2 + 9 b u_a F_a + a Pi_aa
-//   G_ab = 9 rho u_a u_b + 9 b (u_a F_b + u_b F_a) + 2 a Pi_ab      (a < b)
-// with a = 4.5 (1 - omega), b = 1 - omega/2.
-template <int Q, int RHEO, typename T>
-__device__ __forceinline__ void coeffs_collide(T* c, const Moments<Q, RHEO, T>& m, const Force<T>& F) {
-    const T om = m.omega;
-    const T a = (T)4.5 * ((T)1 - om);
-    const T b = (T)1 - (T)0.5 * om;
-    const T uf = m.ux * F.x + m.uy * F.y + m.uz * F.z;
-    const T usq = m.ux * m.ux + m.uy * m.uy + m.uz * m.uz;
-    const T tr = m.pxx + m.pyy + m.pzz;
-    const T r3 = (T)3 * m.rho, r45 = (T)4.5 * m.rho, r9 = (T)9 * m.rho;
-    const T bf = (T)3 * b - a / (T)3, b9 = (T)9 * b, a2 = (T)2 * a;
-    c[0] = m.dr - (T)1.5 * m.rho * usq - a * tr / (T)3 - (T)3 * b * uf;
-    c[1] = r3 * m.ux + bf * F.x;
-    c[2] = r3 * m.uy + bf * F.y;
-    c[3] = r3 * m.uz + bf * F.z;
-    c[4] = r45 * m.ux * m.ux + b9 * m.ux * F.x + a * m.pxx;
-    c[5] = r45 * m.uy * m.uy + b9 * m.uy * F.y + a * m.pyy;
-    c[6] = r45 * m.uz * m.uz + b9 * m.uz * F.z + a * m.pzz;
-    c[7] = r9 * m.ux * m.uy + b9 * (m.ux * F.y + m.uy * F.x) + a2 * m.pxy;
-    c[8] = r9 * m.ux * m.uz + b9 * (m.ux * F.z + m.uz * F.x) + a2 * m.pxz;
-    c[9] = r9 * m.uy * m.uz + b9 * (m.uy * F.z + m.uz * F.y) + a2 * m.pyz;
-}
-
 // ---------------------------------------------------------------------------
 // Kernels
 // ---------------------------------------------------------------------------
 
+// Force on a node: the constant one, or with IBM that of the force field in a
+// flagged tile.
+template <bool IBM, typename T>
+__device__ __forceinline__ Force<T> node_force(const Params<T>& p, const Node<T>& nd) {
+    if (IBM && p.tile_flag[tile_of(p, nd.x, nd.y, nd.z)])
+        return Force<T>{p.ibm_fx[nd.idx], p.ibm_fy[nd.idx], p.ibm_fz[nd.idx]};
+    return const_force(p);
+}
+
 // Moments, apparent omega, saved macroscopics and collision of one node whose
 // post-stream, post-BC deviations are g; the post-collision state goes to
-// dst in representation OUT.
-template <int Q, typename S, int RHEO, bool IBM, int OUT>
+// dst in representation OUT. om_old: the power law's omega of the node.
+template <int Q, typename S, int RHEO, int OUT>
 __device__ __forceinline__ void collide_store(const Params<typename ComputeOf<S>::type>& p, uint32_t idx,
-                                              const Node<typename ComputeOf<S>::type>& nd,
-                                              typename ComputeOf<S>::type* g) {
+                                              typename ComputeOf<S>::type* g,
+                                              const Force<typename ComputeOf<S>::type>& F,
+                                              typename ComputeOf<S>::type om_old) {
     using T = typename ComputeOf<S>::type;
-    Force<T> F = const_force(p);
-    if (IBM && p.tile_flag[tile_of(p, nd.x, nd.y, nd.z)]) F = Force<T>{p.ibm_fx[idx], p.ibm_fy[idx], p.ibm_fz[idx]};
-    const T om_old = (RHEO == 2) ? p.omega_state[idx] : (T)0;
-    const Moments<Q, RHEO, T> m = moments<Q, RHEO, T>(g, p, om_old, F);
+    const Moments<Q, RHEO, T> m = moments<Q, RHEO, kSequential<S>>(g, p, om_old, F);
     if (RHEO == 2) p.omega_state[idx] = m.omega;
     // LES_EXPORT_VISC_TURBULENT: every step, as the reference (lbm.cu:237-239)
     if (RHEO == 0 && p.visc_turb) p.visc_turb[idx] = m.tau_t / (T)3;
@@ -865,6 +1005,7 @@ __device__ __forceinline__ void collide_store(const Params<typename ComputeOf<S>
         return;
     }
     if (p.bgk) collide_bgk<Q, RHEO, T>(g, m, F);
+    else if constexpr (kSequential<S>) collide_seq<Q, RHEO, T>(g, m, F);
     else collide<Q, RHEO, T>(g, m, F);
     if constexpr (sizeof(S) == 2) {
         if (p.sr) {
@@ -902,7 +1043,7 @@ __device__ __forceinline__ void step_node(const Params<typename ComputeOf<S>::ty
         gather<Q, T>(g, pc);
         if (w_scheme(word) != kNull) apply_bc<Q, T, MASK>(g, p, nd, word, pc);
     }
-    collide_store<Q, S, RHEO, IBM, OUT>(p, idx, nd, g);
+    collide_store<Q, S, RHEO, OUT>(p, idx, g, node_force<IBM>(p, nd), RHEO == 2 ? p.omega_state[idx] : (T)0);
 }
 
 // One pulled step of a population node (gather_rows); every thread of the
@@ -950,7 +1091,7 @@ __device__ __forceinline__ void step_node_rows(const Params<typename ComputeOf<S
         if (!in || !w_used(word)) return;
         if (w_scheme(word) != kNull) apply_bc<Q, T, MASK>(g, p, nd, word, GlobalPC<Q, S, T, kRepPop>{p, nd});
     }
-    collide_store<Q, S, RHEO, IBM, OUT>(p, idx, nd, g);
+    collide_store<Q, S, RHEO, OUT>(p, idx, g, node_force<IBM>(p, nd), RHEO == 2 ? p.omega_state[idx] : (T)0);
 }
 
 // One time step over the lattice, one node per thread; ROWS: pull through
@@ -1043,7 +1184,7 @@ __global__ __launch_bounds__(kBlock) void k_aux(const Params<typename ComputeOf<
     }
     if (!w_used(word)) return;
     const T om_old = (RHEO == 2) ? p.omega_state[idx] : (T)0;
-    const Moments<Q, RHEO, T> m = moments<Q, RHEO, T>(g, p, om_old, const_force(p));
+    const Moments<Q, RHEO, T> m = moments<Q, RHEO, kSequential<S>>(g, p, om_old, const_force(p));
     p.m_rho[idx] = m.rho; p.m_ux[idx] = m.ux; p.m_uy[idx] = m.uy; p.m_uz[idx] = m.uz;
     if (RHEO != 0) p.m_omega[idx] = m.omega;
 }
@@ -1076,7 +1217,7 @@ __global__ __launch_bounds__(kBlock) void k_ibm_macr(const Params<typename Compu
             gather<Q, T>(g, pc);
             if (w_scheme(word) != kNull) apply_bc<Q, T, MASK>(g, p, nd, word, pc);
         }
-        const Moments<Q, 0, T> m = moments<Q, 0, T>(g, p, (T)0, const_force(p));
+        const Moments<Q, 0, T> m = moments<Q, 0, kSequential<S>>(g, p, (T)0, const_force(p));
         p.ibm_stage[idx] = StageRec<T>{m.rho, m.ux, m.uy, m.uz};
         ffx[idx] = p.fx; ffy[idx] = p.fy; ffz[idx] = p.fz;
     }

@@ -152,6 +152,7 @@ struct Params {
     uint32_t sr_seed;           // its random stream of this step
     int aux_f64;                // kAuxMaterialize: doubles into dst, planes of aux_count values
     T duct_R, duct_r, w_out, u_out, w_in, u_in;
+    const T* ibb;               // interpolated bounce-back weights: outer wall, then inner, 8 planes of nx * ny each
     // immersed boundary: nodes in 8^3 tiles flagged by the last IBM stage take
     // their force from ibm_f*, every other node the constant (fx, fy, fz)
     const uint32_t* tile_flag;
@@ -207,6 +208,7 @@ int launch_reduce(int prec, const void* rho, const void* ux, const void* uy, con
                   void* uy_old, void* uz_old, uint32_t n, double* partials, double* out3, void* stream);
 int launch_fill_feq(int q, int prec, void* state, int64_t stride, uint32_t n, const double* rho,
                     const double* ux, const double* uy, const double* uz, void* stream, int out_rep = 0);
+int launch_ibb_table(int prec, const void* params, void* table, void* stream);
 int launch_convert(int prec, void* buf, double* dbl, size_t count, int to_double, void* stream);
 int launch_copy_probe(const void* src, void* dst, size_t bytes, void* stream);
 
