@@ -95,3 +95,11 @@ def test_node_maps(vel_set, builder, precision):
 def test_immersed_boundary_force(builder, vel_set, precision):
     for rheology in RHEOLOGY.values():
         compare((24, 24, 20), precision, vel_set, ibm=True, builder=builder, **rheology)
+
+
+@pytest.mark.parametrize("size,precision", [((70, 66, 60), "single"), ((66, 50, 50), "double")])
+def test_population_step_through_the_caches(size, precision):
+    """Lattices from 40 MB (two of 19 planes) on store through the caches and run every other step from the last
+    block to the first; the block counts here are no multiples of 8, so some blocks stay where they are."""
+    compare(size, precision, **BOX["duct"], **RHEOLOGY["bingham"])
+    compare(size, precision, ibm=True, **BOX["closed"], **RHEOLOGY["newtonian"])

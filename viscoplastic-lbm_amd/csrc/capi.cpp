@@ -742,6 +742,7 @@ static int enqueue_steps(vlbm_h h, int n_steps, int save_last, hipEvent_t* ev = 
             // IBM builds take the macroscopics from the stage (save_macr_to_array
             // is false with IBM, src/CUDA/main.cu:293-297)
             p.save = (save && !ibm) ? 1 : 0;
+            p.odd = (int)(h->steps & 1);
             p.sr_seed = (uint32_t)h->steps * 0x9e3779b9u + 0x7f4a7c15u;
             return check_launch(launch_step(d.q, d.precision, d.rheology, h->mask_geom, h->direct, pv, h->stream, ibm,
                                             state_rep(h), h->mom ? kRepMom : kRepPop),

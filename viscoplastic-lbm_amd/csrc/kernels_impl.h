@@ -64,6 +64,7 @@ template <> __device__ __forceinline__ float ld_nt<bf16, float>(const bf16* p) {
     return __uint_as_float((uint32_t)__builtin_nontemporal_load((const uint16_t*)p) << 16);
 }
 
+template <typename S, typename T> __device__ __forceinline__ void st(S* p, T v) { *p = (S)v; }
 template <typename S, typename T> __device__ __forceinline__ void st_nt(S* p, T v) {
     __builtin_nontemporal_store((S)v, p);
 }
@@ -585,6 +586,16 @@ template <int Q> struct XShifted {
     }
 };
 
+// Block of nodes a workgroup takes. Cached steps (Params::cached) go back and
+// forth through the lattice, so that what the step before wrote last is read
+// first. Blocks keep their residue mod 8, the XCD they run on.
+template <typename T>
+__device__ __forceinline__ uint32_t step_block(const Params<T>& p) {
+    const uint32_t octets = gridDim.x / 8u, o = blockIdx.x / 8u;
+    if (!p.cached || !p.odd || o >= octets) return blockIdx.x;
+    return (octets - 1u - o) * 8u + blockIdx.x % 8u;
+}
+
 template <int Q, typename S, typename T>
 __device__ __forceinline__ void gather_rows(T* g, const Params<T>& p, const Node<T>& nd, T* sm) {
     const int t = (int)threadIdx.x;
@@ -1020,6 +1031,15 @@ __device__ __forceinline__ void collide_store(const Params<typename ComputeOf<S>
             return;
         }
     }
+    if (sizeof(S) > 2 && p.cached) {
+        // the empty asm keeps the compiler from merging the two branches into
+        // one set of stores, which drops the non-temporal hint
+        asm volatile("");
+#pragma unroll
+        for (int i = 0; i < Q; i++) st<S, T>(dst + (int64_t)i * p.stride + idx, g[i]);
+        asm volatile("");
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < Q; i++) st_nt<S, T>(dst + (int64_t)i * p.stride + idx, g[i]);
 }
@@ -1100,7 +1120,7 @@ template <int Q, typename S, int RHEO, bool MASK, bool DIRECT, bool IBM = false,
           bool ROWS = false>
 __global__ __launch_bounds__(kBlock) void k_step(const Params<typename ComputeOf<S>::type> p) {
     static_assert(!ROWS || (!DIRECT && IN == kRepPop), "the row pull reads populations of the previous step");
-    const uint32_t idx = blockIdx.x * kBlock + threadIdx.x;
+    const uint32_t idx = (ROWS ? blockIdx.x : step_block(p)) * kBlock + threadIdx.x;
     if constexpr (ROWS) {
         __shared__ typename ComputeOf<S>::type sm[XShifted<Q>::count() * kBlock];
         const bool in = idx < p.n;                            // the grid holds no block wholly past the lattice

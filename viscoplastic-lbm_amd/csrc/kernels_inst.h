@@ -34,6 +34,15 @@ struct Inst {
         }
     }
 
+    // Whether a population step of two lattices of `bytes` in all stores through
+    // the caches (256 MB memory-side cache, 8 x 4 MB L2) and runs back and forth,
+    // instead of streaming past them. D3Q19, us a step, streaming and cached:
+    // 30 MB 7.2 7.8, 56 MB 14.4 12.1, 134 MB 28.4 23.9, 237 MB 45.8 40.2,
+    // 398 MB 78.5 74.7, 456 MB 95.0 87.3, 840 MB (double) 158 157. Below, the
+    // write-back at the kernel's end costs more; above, little is left of the
+    // step before. The row pull keeps streaming (80 MB 18.1 19.5, 319 MB 65.1 68.8).
+    static int cached_step(double bytes) { return bytes >= 40e6 && bytes <= 512e6 ? 1 : 0; }
+
     template <int Q, int RHEO, bool MASK, bool IBM>
     static void step_pop(bool direct, const Params<T>& p, hipStream_t st) {
         if (direct) {
@@ -48,7 +57,9 @@ struct Inst {
                 return;
             }
         }
-        hipLaunchKernelGGL((k_step<Q, S, RHEO, MASK, false, IBM>), grid_of(p.n), dim3(kBlock), 0, st, p);
+        Params<T> pc = p;
+        pc.cached = cached_step(2.0 * Q * sizeof(S) * p.n);
+        hipLaunchKernelGGL((k_step<Q, S, RHEO, MASK, false, IBM>), grid_of(p.n), dim3(kBlock), 0, st, pc);
     }
 
     template <int Q, int RHEO>
