@@ -40,6 +40,7 @@ SOURCES = [
     "kernels_batch.hip",
     "batch_capi.cpp",
     "checkpoint.cpp",
+    "host_copy.cpp",
     "capi.cpp",
     "noalloc.hip",
 ]

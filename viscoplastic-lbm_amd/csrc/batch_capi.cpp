@@ -21,6 +21,8 @@
 #include <cstring>
 #include <deque>
 #include <map>
+#include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -49,7 +51,9 @@ struct Job {
     int phase = 0;
     long long next_check = 0;
     bool has_result = false;
-    std::vector<double> res[4];
+    std::unique_ptr<char[]> res;               // rho, ux, uy, uz in the compute type, one after the other
+    size_t res_bytes = 0;
+    size_t nodes() const { return (size_t)d.nx * d.ny * d.nz; }
 };
 
 }  // namespace
@@ -83,6 +87,10 @@ struct vlbm_batch {
     std::string tuned_key;                     // resident-node bucket the launch shape was chosen for
     bool fixed_shape = false;                  // K, block and grid given by the caller
     std::map<std::string, std::array<int, 3>> shapes;   // launch shapes chosen in this batch, by key
+    std::multimap<size_t, std::unique_ptr<char[]>> spare;   // released result buffers by size
+    size_t spare_bytes = 0;
+    HostCopy host_copy;                        // staging of the result downloads
+    int device = 0;                            // device current at vlbm_batch_create (the stream's device)
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     int graph_K = 0, graph_block = 0, graph_grid = 0, graph_rheo = -1;
@@ -247,6 +255,34 @@ int admit(vlbm_batch* b, int id) {
     return VLBM_OK;
 }
 
+// Result buffers. Released ones are kept for later jobs, at most kSpareBytes of
+// them in a batch: a fresh buffer costs its page faults, as much time as its copy.
+constexpr size_t kSpareBytes = size_t(256) << 20;
+
+int take_result(vlbm_batch* b, Job& j, size_t bytes) {
+    auto best = b->spare.lower_bound(bytes);
+    if (best != b->spare.end() && best->first <= 2 * bytes) {
+        j.res_bytes = best->first;
+        j.res = std::move(best->second);
+        b->spare_bytes -= best->first;
+        b->spare.erase(best);
+        return VLBM_OK;
+    }
+    j.res.reset(new (std::nothrow) char[bytes]);
+    if (!j.res) return fail(VLBM_ERR_ALLOC, "result of a job: host allocation failed");
+    j.res_bytes = bytes;
+    return VLBM_OK;
+}
+
+void give_result(vlbm_batch* b, Job& j) {
+    if (j.res && b->spare_bytes + j.res_bytes <= kSpareBytes) {
+        b->spare_bytes += j.res_bytes;
+        b->spare.emplace(j.res_bytes, std::move(j.res));
+    }
+    j.res.reset();
+    j.res_bytes = 0;
+}
+
 // final macroscopics into the idle lattice of the job, then to the host
 int retire(vlbm_batch* b, int id, int state) {
     Job& j = b->jobs[id];
@@ -273,17 +309,10 @@ int retire(vlbm_batch* b, int id, int state) {
         rc = launch_aux(j.d.q, j.d.precision, j.d.rheology, false, &p, b->stream);
     }
     if (rc) return check_launch(rc, "final moments");
-    std::vector<char> host(4 * fb);
-    HIP_TRY(hipMemcpyAsync(host.data(), idle, 4 * fb, hipMemcpyDeviceToHost, b->stream));
-    if ((rc = sync(b))) return rc;
-    for (int f = 0; f < 4; f++) {
-        j.res[f].resize(n);
-        if (b->tbytes == 8) std::memcpy(j.res[f].data(), host.data() + f * fb, fb);
-        else {
-            const float* src = (const float*)(host.data() + f * fb);
-            for (size_t k = 0; k < n; k++) j.res[f][k] = src[k];
-        }
-    }
+    if ((rc = take_result(b, j, 4 * fb))) return rc;
+    FieldCopy fields[4];
+    for (int f = 0; f < 4; f++) fields[f] = FieldCopy{idle + f * fb, j.res.get() + f * fb};
+    HIP_TRY(b->host_copy.fetch(b->device, b->stream, fields, 4, n, b->tbytes, true));
     j.has_result = true;
     j.state = state;
     j.t_end = b->now();
@@ -585,6 +614,7 @@ int vlbm_batch_create(const vlbm_batch_desc* d, vlbm_batch_h* out) {
         vlbm_batch_destroy(b);
         return fail(code, m);
     };
+    if (hipGetDevice(&b->device) != hipSuccess) return bail(VLBM_ERR_DEVICE, "hipGetDevice failed");
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) return bail(VLBM_ERR_DEVICE, "hipStreamCreate failed");
     b->arena_bytes = d->hbm_budget / kAlign * kAlign;
     if (hipMalloc((void**)&b->arena, b->arena_bytes) != hipSuccess) {
@@ -715,8 +745,9 @@ int vlbm_batch_job_result(vlbm_batch_h b, int job, double* rho, double* ux, doub
     const Job& j = b->jobs[job];
     if (!j.has_result) return fail(VLBM_ERR_INVALID, "job has no result (still running, or released)");
     double* outs[4] = {rho, ux, uy, uz};
+    const size_t n = j.nodes();
     for (int f = 0; f < 4; f++)
-        if (outs[f]) std::memcpy(outs[f], j.res[f].data(), j.res[f].size() * sizeof(double));
+        if (outs[f]) widen(outs[f], j.res.get() + f * n * b->tbytes, n, b->tbytes);
     return VLBM_OK;
 }
 
@@ -725,7 +756,7 @@ int vlbm_batch_release(vlbm_batch_h b, int job) {
     if (rc) return rc;
     if (job < 0 || job >= (int)b->jobs.size()) return fail(VLBM_ERR_INVALID, "unknown job");
     Job& j = b->jobs[job];
-    for (auto& v : j.res) std::vector<double>().swap(v);
+    give_result(b, j);
     j.has_result = false;
     return VLBM_OK;
 }

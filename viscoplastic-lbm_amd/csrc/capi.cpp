@@ -838,13 +838,14 @@ int vlbm_compute_macroscopics(vlbm_h h) {
 int vlbm_macroscopics(vlbm_h h, double* rho, double* ux, double* uy, double* uz, double* omega) {
     if (!h) return fail(VLBM_ERR_INVALID, "handle is NULL");
     double* outs[5] = {rho, ux, uy, uz, omega};
+    FieldCopy fields[5];
+    int count = 0;
     for (int k = 0; k < 5; k++) {
         if (!outs[k]) continue;
         if (!h->macr[k]) return fail(VLBM_ERR_INVALID, "omega exists for non-Newtonian fluids only");
-        int rc = fetch_field(h, h->macr[k], outs[k]);
-        if (rc) return rc;
+        fields[count++] = FieldCopy{h->macr[k], outs[k]};
     }
-    return VLBM_OK;
+    return fetch_fields(h, fields, count);
 }
 
 int vlbm_visc_turb(vlbm_h h, double* out) {

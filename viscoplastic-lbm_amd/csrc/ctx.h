@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/vlbm.h"
+#include "host_copy.h"
 #include "lattice.h"
 
 namespace vlbm {
@@ -69,6 +70,7 @@ struct vlbm_ctx {
     int device = 0;           // device current at vlbm_create (the stream's device)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     size_t device_bytes = 0;
+    vlbm::detail::HostCopy host_copy;   // staging of the field downloads
     vlbm::IbmState* ibm = nullptr;   // immersed boundary stage (vlbm_ibm_enable)
     // what the step kernel needs of the IBM stage (null without IBM)
     const uint32_t* tile_flag = nullptr;
@@ -202,18 +204,15 @@ inline int dalloc(vlbm_ctx* h, void** p, size_t bytes) {
     return VLBM_OK;
 }
 
-// Host copy of a macroscopic field (compute type) as doubles.
-inline int fetch_field(vlbm_ctx* h, const void* dev, double* out) {
-    if (h->tbytes == 8) {
-        HIP_TRY(hipMemcpyAsync(out, dev, h->n * 8, hipMemcpyDeviceToHost, h->stream));
-        HIP_TRY(hipStreamSynchronize(h->stream));
-        return VLBM_OK;
-    }
-    std::vector<float> tmp(h->n);
-    HIP_TRY(hipMemcpyAsync(tmp.data(), dev, h->n * 4, hipMemcpyDeviceToHost, h->stream));
-    HIP_TRY(hipStreamSynchronize(h->stream));
-    for (size_t k = 0; k < h->n; k++) out[k] = tmp[k];
+// Host copies of fields (compute type) as doubles.
+inline int fetch_fields(vlbm_ctx* h, const FieldCopy* fields, int count) {
+    HIP_TRY(h->host_copy.fetch(h->device, h->stream, fields, count, h->n, h->tbytes));
     return VLBM_OK;
+}
+
+inline int fetch_field(vlbm_ctx* h, const void* dev, double* out) {
+    const FieldCopy f{dev, out};
+    return fetch_fields(h, &f, 1);
 }
 
 inline int upload_field(vlbm_ctx* h, void* dev, const double* in) {

@@ -1,0 +1,170 @@
+// Field downloads (host_copy.h).
+#include "host_copy.h"
+
+#include <sched.h>
+
+#include <algorithm>
+#include <atomic>
+#include <condition_variable>
+#include <cstdlib>
+#include <cstring>
+#include <thread>
+
+namespace vlbm {
+namespace detail {
+namespace {
+
+constexpr int kThreads = 4;
+
+// CPUs this process may run on.
+int cpus() {
+    cpu_set_t set;
+    CPU_ZERO(&set);
+    if (sched_getaffinity(0, sizeof(set), &set) == 0) return std::max(1, CPU_COUNT(&set));
+    return std::max(1u, std::thread::hardware_concurrency());
+}
+
+// fn(0) on this thread, after fn(1) ... fn(workers - 1) have been started on
+// their own; fewer when the system refuses a thread. fn must not need them all.
+template <typename F>
+void run_workers(int workers, F&& fn) {
+    std::thread threads[kThreads];
+    int started = 0;
+    try {
+        for (int w = 1; w < workers && w < kThreads; w++) {
+            threads[started] = std::thread([&fn, w] { fn(w); });
+            started++;
+        }
+    } catch (...) {
+    }
+    fn(0);
+    for (int t = 0; t < started; t++) threads[t].join();
+}
+
+}  // namespace
+
+void widen(double* out, const void* in, size_t n, int value_bytes) {
+    if (value_bytes == 8) {
+        std::memcpy(out, in, n * 8);
+        return;
+    }
+    const float* f = (const float*)in;
+    for (size_t k = 0; k < n; k++) out[k] = f[k];
+}
+
+hipError_t HostCopy::reserve(int slots, size_t bytes) {
+    slots = std::min(slots, kSlots);
+    if (bytes > slot_bytes_) {
+        release();
+        slot_bytes_ = bytes;
+    }
+    for (; slots_ < slots; slots_++) {
+        void* p = nullptr;
+        pinned_[slots_] = hipHostMalloc(&p, slot_bytes_, hipHostMallocDefault) == hipSuccess;
+        if (!pinned_[slots_]) {
+            // pageable memory carries the same copy, staged by the runtime
+            (void)hipGetLastError();
+            p = std::malloc(slot_bytes_);
+            if (!p) break;
+        }
+        if (hipEventCreateWithFlags(&event_[slots_], hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            if (pinned_[slots_]) (void)hipHostFree(p);
+            else std::free(p);
+            break;
+        }
+        slot_[slots_] = p;
+    }
+    return slots_ ? hipSuccess : hipErrorOutOfMemory;
+}
+
+void HostCopy::release() {
+    for (int k = 0; k < slots_; k++) {
+        (void)hipEventDestroy(event_[k]);
+        if (pinned_[k]) (void)hipHostFree(slot_[k]);
+        else std::free(slot_[k]);
+        slot_[k] = nullptr;
+    }
+    slots_ = 0;
+    slot_bytes_ = 0;
+}
+
+hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fields, int count, size_t n,
+                           int value_bytes, bool raw) {
+    std::lock_guard<std::mutex> lock(mu_);
+    const size_t vb = (size_t)value_bytes, total = n * (size_t)count * vb;
+    // slots of 2 MB with threads, of 512 KB without (the first copy, which nothing overlaps, is shorter)
+    const bool threads = total >= (size_t(16) << 20);
+    const size_t per = std::min(n, (threads ? kSlotBytes : kSlotBytes / 4) / vb);        // values of a chunk
+    const size_t per_field = per ? (n + per - 1) / per : 0, chunks = per_field * (size_t)count;
+    if (!chunks) return hipSuccess;
+    hipError_t e = reserve((int)std::min<size_t>(chunks, kSlots), per * vb);
+    if (e != hipSuccess) return e;
+    struct Chunk { const char* dev; char* out; size_t n; };
+    const size_t ob = raw ? vb : sizeof(double);
+    auto chunk = [&](size_t i) {
+        const FieldCopy& f = fields[i / per_field];
+        const size_t at = i % per_field * per;
+        return Chunk{(const char*)f.dev + at * vb, (char*)f.out + at * ob, std::min(per, n - at)};
+    };
+    auto enqueue = [&](size_t i, int s) {
+        const Chunk c = chunk(i);
+        const hipError_t ec = hipMemcpyAsync(slot_[s], c.dev, c.n * vb, hipMemcpyDeviceToHost, stream);
+        return ec == hipSuccess ? hipEventRecord(event_[s], stream) : ec;
+    };
+    auto finish = [&](size_t i, int s) {
+        const hipError_t es = hipEventSynchronize(event_[s]);
+        if (es != hipSuccess) return es;
+        const Chunk c = chunk(i);
+        if (raw) std::memcpy(c.out, slot_[s], c.n * vb);
+        else widen((double*)c.out, slot_[s], c.n, value_bytes);
+        return hipSuccess;
+    };
+    if (!threads) {
+        const size_t ahead = (size_t)slots_;
+        for (size_t i = 0; i < std::min(ahead, chunks) && e == hipSuccess; i++) e = enqueue(i, (int)i);
+        for (size_t i = 0; i < chunks && e == hipSuccess; i++) {
+            e = finish(i, (int)(i % ahead));
+            if (e == hipSuccess && i + ahead < chunks) e = enqueue(i + ahead, (int)(i % ahead));
+        }
+        if (e != hipSuccess) (void)hipStreamSynchronize(stream);      // no copy into a slot outlives the call
+        return e;
+    }
+    std::atomic<size_t> touch{0}, next{0};
+    std::atomic<int> error{(int)hipSuccess};
+    std::atomic<bool> ready{false};
+    std::mutex m;
+    std::condition_variable cv;
+    auto worker = [&](int w) {
+        hipError_t we = hipSuccess;
+        if (w == 0) {
+            we = hipStreamSynchronize(stream);
+            {
+                std::lock_guard<std::mutex> g(m);
+                ready = true;
+            }
+            cv.notify_all();
+        } else {
+            we = hipSetDevice(device);
+            // the pages of the destination, while the stream computes
+            for (size_t i; !ready && (i = touch++) < chunks;) {
+                const Chunk c = chunk(i);
+                for (size_t k = 0; k < c.n * ob && !ready; k += 4096) *(volatile char*)(c.out + k) = 0;
+            }
+            std::unique_lock<std::mutex> g(m);
+            cv.wait(g, [&] { return ready.load(); });
+        }
+        for (size_t i; we == hipSuccess && error == (int)hipSuccess && (i = next++) < chunks;) {
+            we = enqueue(i, w);
+            if (we == hipSuccess) we = finish(i, w);
+        }
+        if (we != hipSuccess) error = (int)we;
+    };
+    run_workers(std::min({slots_, kThreads, cpus()}), worker);
+    // a copy of a worker that stopped early may still be under way into its slot
+    if (error != (int)hipSuccess) (void)hipStreamSynchronize(stream);
+    return (hipError_t)error.load();
+}
+
+}  // namespace detail
+}  // namespace vlbm

@@ -1,0 +1,60 @@
+// Download of fields from the device.
+//
+// What bounds it is the host: the link carries 55 GB/s, while one thread that
+// lets the runtime stage a pageable copy into a fresh temporary and then
+// converts it writes every page three times and faults it in twice (four
+// fields of a 256^3 float lattice: 107 ms, of which the link needs 5). Here the
+// copies go into page-locked slots and are converted from there into place. From
+// 16 MB on, 4 threads each take the next chunk, so the page faults and
+// conversions of different chunks overlap, and while the stream still computes
+// they fault in the destination: 17 ms for those fields after an idle stream (8
+// threads 14, 2 27, 1 45), about 8 behind 200 steps. Below, one thread with all
+// slots in flight: threads gain little there and get in the way of a caller's own
+// pool (four fields of 0.6 million nodes between torch operations: 2 to 6 ms with
+// 4 threads, 1.4 with one).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <mutex>
+
+namespace vlbm {
+namespace detail {
+
+struct FieldCopy {
+    const void* dev;      // n values of 4 or 8 bytes on the device
+    void* out;            // on the host: n doubles, or n values as they are on the device
+};
+
+// Page-locked staging of one owner (a lattice handle, a batch): at most 8
+// slots of 2 MB, allocated by the first download that needs them and freed
+// with the owner. Downloads of one owner from several threads take turns.
+class HostCopy {
+public:
+    HostCopy() = default;
+    HostCopy(const HostCopy&) = delete;
+    HostCopy& operator=(const HostCopy&) = delete;
+    ~HostCopy() { release(); }
+    // The fields, after everything enqueued on the stream so far; returns when they are in place. As doubles, or
+    // raw as they are on the device.
+    hipError_t fetch(int device, hipStream_t stream, const FieldCopy* fields, int count, size_t n, int value_bytes,
+                     bool raw = false);
+    void release();
+
+private:
+    static constexpr int kSlots = 8;
+    static constexpr size_t kSlotBytes = size_t(2) << 20;
+    hipError_t reserve(int slots, size_t bytes);
+    std::mutex mu_;
+    void* slot_[kSlots] = {};
+    bool pinned_[kSlots] = {};
+    hipEvent_t event_[kSlots] = {};
+    size_t slot_bytes_ = 0;
+    int slots_ = 0;
+};
+
+// out[k] = in[k] for n values of 4 or 8 bytes.
+void widen(double* out, const void* in, size_t n, int value_bytes);
+
+}  // namespace detail
+}  // namespace vlbm
