@@ -980,11 +980,19 @@ __global__ __launch_bounds__(kInterpBlock) void k_ibm_spread(IbmParams P, IbmFlu
     add_spread<T>(fl, kk, (T)(-P.pdx[i] * pt.a), (T)(-P.pdy[i] * pt.a), (T)(-P.pdz[i] * pt.a));
 }
 
-// (2b) FP32 fluids: one workgroup per sphere, 16 lanes per node (one stencil
-// row each), collects the spread force in an LDS box of edge^3 nodes around
-// the sphere and adds the box to the force field and the stage velocities
-// with one global atomic per box node, field and component. Points outside
-// the box (nodes that left the sphere's radius) go straight to global memory.
+// (2b) FP32 fluids: a workgroup per z-slab of a sphere's box of edge^3 nodes
+// (16 lanes per node, one stencil row each) collects the spread force of the
+// slab in LDS and adds it to the force field and the stage velocities with one
+// global atomic per box node, field and component. Points outside the box
+// (nodes that left the sphere's radius) go straight to global memory, by the
+// first slab. The slabs of a sphere scale alike (box_slabs): every one sums the
+// sphere's forces in the same order.
+//
+// What bounds it is latency: LDS atomics, then dependent loads and stores of the
+// flush. With one workgroup per sphere a suspension of a few dozen spheres leaves
+// most CUs idle, and each workgroup flushes a whole box. 48 spheres of radius 8
+// (804 nodes): 57 us a launch that way, 29 now (of that 8 from the flush no longer
+// working out neighbours of empty places).
 //
 // The box holds fixed-point integers (LDS integer atomics; float LDS atomics
 // cost several times more): component a of a contribution -dF_a w is stored
@@ -996,29 +1004,36 @@ __global__ __launch_bounds__(kInterpBlock) void k_ibm_spread(IbmParams P, IbmFlu
 // contribution is at most 2^-31 of the sphere's force sum. A sphere whose
 // force sum is not finite spreads through the global float atomics, so that
 // the fluid sees the same NaN or infinity as the sphere.
+constexpr int kSpreadBatch = 512;     // nodes; 24 KB beside a whole box of at most 128 KB
 __device__ __forceinline__ int box_fixed(double v, double s) { return (int)rint(v * s); }
 
 __global__ __launch_bounds__(kSphereBlock) void k_ibm_spread_box(IbmParams P, IbmFluid<float> fl) {
-    extern __shared__ int box[];                   // [3][edge^3]
+    extern __shared__ int box[];                   // [3][slab planes][edge^2]
+    __shared__ double kept[6 * kSpreadBatch];      // position and force of the batch's nodes for this slab
+    __shared__ int n_kept;
     __shared__ double red[3][kSphereBlock / 64];
     __shared__ double scale[3];
     __shared__ int finite[3];
     __shared__ int nb_o[kBoxNb][3];                // origins of the overlapping boxes
-    const IbmSphere& c = P.sph[blockIdx.x];
-    const int* plan = P.box_nb + blockIdx.x * (kBoxNb + 1);
+    const int sphere = (int)blockIdx.x;
+    const IbmSphere& c = P.sph[sphere];
+    const int* plan = P.box_nb + sphere * (kBoxNb + 1);
     const int n_nb = P.box_plain && *P.box_stray == 0 ? plan[0] : -1;   // -1: atomics everywhere
     if ((int)threadIdx.x < n_nb) {
         const IbmSphere& cj = P.sph[plan[1 + threadIdx.x]];
         for (int a = 0; a < 3; a++) nb_o[threadIdx.x][a] = box_origin(P, cj, a);
     }
     const int edge = P.box_edge;
-    const int e3 = edge * edge * edge;
+    const int per = (edge + (int)gridDim.y - 1) / (int)gridDim.y;       // planes of a slab
+    const int s0 = (int)blockIdx.y * per, planes = min(per, edge - s0); // this one's: [s0, s0 + planes)
+    const bool first_slab = blockIdx.y == 0;
+    if (planes <= 0) return;
+    const int e3 = planes * edge * edge;
     for (int e = threadIdx.x; e < 3 * e3; e += kSphereBlock) box[e] = 0;
     const int half = edge / 2 - 3;                 // ceil(radius)
     int o[3];
     for (int a = 0; a < 3; a++) o[a] = (int)floor(c.pos[a]) - half - 2;
     const int first = c.first_node;
-    const int items = c.n_nodes * kRowLanes;
     {
         double sa[3] = {0, 0, 0};
         for (int k = threadIdx.x; k < c.n_nodes; k += kSphereBlock) {
@@ -1038,55 +1053,79 @@ __global__ __launch_bounds__(kSphereBlock) void k_ibm_spread_box(IbmParams P, Ib
     }
     const int r = threadIdx.x & (kRowLanes - 1);
     const int zk = r >> 2, yj = r & 3;
-    // position and force of the node of item k (the sphere's first node past
-    // the end); the next item's are loaded while the current one is spread
-    auto fetch = [&](int k, double (&q)[6]) {
-        const int i = first + (k < items ? k / kRowLanes : 0);
-        q[0] = P.px[i]; q[1] = P.py[i]; q[2] = P.pz[i];
-        q[3] = P.pdx[i]; q[4] = P.pdy[i]; q[5] = P.pdz[i];
-    };
-    double nxt[6] = {0, 0, 0, 0, 0, 0};
-    if (items > 0) fetch((int)threadIdx.x, nxt);
     __syncthreads();
     const double sx = scale[0], sy = scale[1], sz = scale[2];
     const bool use_box = finite[0] && finite[1] && finite[2];
-    for (int b0 = 0; b0 < items; b0 += kSphereBlock) {      // uniform trip count for the shuffles
+    // Batches of nodes: the threads read one node each and keep those with a
+    // row for this slab in LDS; then 16 lanes spread each of them.
+    for (int b0 = 0; b0 < c.n_nodes; b0 += kSpreadBatch) {
+        if (threadIdx.x == 0) n_kept = 0;
+        __syncthreads();
         const int k = b0 + (int)threadIdx.x;
-        const bool act = k < items;
         double q[6];
+        bool keep = false;
+        if (threadIdx.x < kSpreadBatch && k < c.n_nodes) {
+            const int i = first + k;
+            q[0] = P.px[i]; q[1] = P.py[i]; q[2] = P.pz[i];
+            q[3] = P.pdx[i]; q[4] = P.pdy[i]; q[5] = P.pdz[i];
+            const double pos[3] = {q[0], q[1], q[2]};
+            const Stencil st = make_stencil(P, pos);
+            // the whole stencil in the box, and planes of it in the slab
+            bool inside = use_box, touches = false;
+            for (int a = 0; a < 3; a++)
+                for (int j = 0; j < 4; j++) {
+                    int d = st.base[a] + j - o[a];
+                    if (P.periodic[a]) d = wrap_axis(d, axis_n(P, a));
+                    inside = inside && d >= 0 && d < edge;
+                    if (a == 2) touches = touches || (d >= s0 && d < s0 + planes);
+                }
+            keep = st.valid && ((use_box && touches) || (first_slab && !inside));
+        }
+        const uint64_t m = __ballot(keep);
+        int at = 0;
+        if ((threadIdx.x & 63) == 0 && m) at = atomicAdd(&n_kept, (int)__popcll(m));
+        at = __shfl(at, 0, 64) + (int)__popcll(m & ((1ull << (threadIdx.x & 63)) - 1ull));
+        if (keep)
+            for (int j = 0; j < 6; j++) kept[j * kSpreadBatch + at] = q[j];
+        __syncthreads();
+        const int items = n_kept * kRowLanes;
+        for (int it0 = 0; it0 < items; it0 += kSphereBlock) {      // uniform trip count for the shuffles
+            const int it = it0 + (int)threadIdx.x;
+            const bool act = it < items;
+            double v[6];
+            for (int j = 0; j < 6; j++) v[j] = kept[j * kSpreadBatch + (act ? it / kRowLanes : 0)];
+            const double pos[3] = {v[0], v[1], v[2]};
+            const Stencil st = make_stencil(P, pos);
+            const RowWeights rw = row_weights(st.base[0], st.base[1], st.base[2], pos[0], pos[1], pos[2], act, r);
+            if (!act || zk < st.mn[2] || zk > st.mx[2] || yj < st.mn[1] || yj > st.mx[1]) continue;
+            const double a1 = rw.zy;
+            const int cz = stencil_coord(P, st, 2, zk), cy = stencil_coord(P, st, 1, yj);
+            int bz = st.base[2] + zk - o[2], by = st.base[1] + yj - o[1];
+            if (P.periodic[2]) bz = wrap_axis(bz, P.nz);
+            if (P.periodic[1]) by = wrap_axis(by, P.ny);
+            const bool in_zy = use_box && by >= 0 && by < edge && bz >= 0 && bz < edge;
+            const bool mine = in_zy && bz >= s0 && bz < s0 + planes;
+            if (!mine && !first_slab) continue;
 #pragma unroll
-        for (int j = 0; j < 6; j++) q[j] = nxt[j];
-        if (b0 + kSphereBlock < items) fetch(k + kSphereBlock, nxt);
-        const double pos[3] = {q[0], q[1], q[2]};
-        Stencil st;
-        st.valid = false;
-        if (act) st = make_stencil(P, pos);
-        const RowWeights rw = row_weights(st.base[0], st.base[1], st.base[2], pos[0], pos[1], pos[2], act && st.valid, r);
-        if (!act || !st.valid || zk < st.mn[2] || zk > st.mx[2] || yj < st.mn[1] || yj > st.mx[1]) continue;
-        const double a1 = rw.zy;
-        const int cz = stencil_coord(P, st, 2, zk), cy = stencil_coord(P, st, 1, yj);
-        int bz = st.base[2] + zk - o[2], by = st.base[1] + yj - o[1];
-        if (P.periodic[2]) bz = wrap_axis(bz, P.nz);
-        if (P.periodic[1]) by = wrap_axis(by, P.ny);
-#pragma unroll
-        for (int xi = 0; xi < 4; xi++) {
-            if (xi < st.mn[0] || xi > st.mx[0]) continue;
-            const double a = a1 * rw.x[xi];
-            const float vx = (float)(-q[3] * a), vy = (float)(-q[4] * a), vz = (float)(-q[5] * a);
-            int bx = st.base[0] + xi - o[0];
-            if (P.periodic[0]) bx = wrap_axis(bx, P.nx);
-            if (use_box && bx >= 0 && bx < edge && by >= 0 && by < edge && bz >= 0 && bz < edge) {
-                const int e = (bz * edge + by) * edge + bx;
-                atomicAdd(box + e, box_fixed(-q[3] * a, sx));
-                atomicAdd(box + e3 + e, box_fixed(-q[4] * a, sy));
-                atomicAdd(box + 2 * e3 + e, box_fixed(-q[5] * a, sz));
-            } else {
-                const size_t kk = ((size_t)cz * P.ny + cy) * P.nx + stencil_coord(P, st, 0, xi);
-                add_spread<float>(fl, kk, vx, vy, vz);
+            for (int xi = 0; xi < 4; xi++) {
+                if (xi < st.mn[0] || xi > st.mx[0]) continue;
+                const double a = a1 * rw.x[xi];
+                int bx = st.base[0] + xi - o[0];
+                if (P.periodic[0]) bx = wrap_axis(bx, P.nx);
+                if (in_zy && bx >= 0 && bx < edge) {
+                    if (!mine) continue;
+                    const int e = ((bz - s0) * edge + by) * edge + bx;
+                    atomicAdd(box + e, box_fixed(-v[3] * a, sx));
+                    atomicAdd(box + e3 + e, box_fixed(-v[4] * a, sy));
+                    atomicAdd(box + 2 * e3 + e, box_fixed(-v[5] * a, sz));
+                } else if (first_slab) {
+                    const size_t kk = ((size_t)cz * P.ny + cy) * P.nx + stencil_coord(P, st, 0, xi);
+                    add_spread<float>(fl, kk, (float)(-v[3] * a), (float)(-v[4] * a), (float)(-v[5] * a));
+                }
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
     // flush in rounds of kFlushBatch box nodes per thread. A node that no
     // other sphere's box covers (and, with use_box, no other workgroup
     // writes: see box_plan) takes plain loads and stores, the others
@@ -1094,7 +1133,7 @@ __global__ __launch_bounds__(kSphereBlock) void k_ibm_spread_box(IbmParams P, Ib
     // the same either way. The loads of a round are issued before its
     // atomics and stores, so each waits for the previous round's only
     // (memory operations retire in order).
-    constexpr int kFlushBatch = 8;
+    constexpr int kFlushBatch = 4;
     const bool plain_ok = use_box && n_nb >= 0;
     for (int e0 = 0; e0 < e3; e0 += kFlushBatch * kSphereBlock) {
         size_t kk[kFlushBatch];
@@ -1105,16 +1144,21 @@ __global__ __launch_bounds__(kSphereBlock) void k_ibm_spread_box(IbmParams P, Ib
         for (int j = 0; j < kFlushBatch; j++) {
             const int e = e0 + j * kSphereBlock + (int)threadIdx.x;
             on[j] = e < e3 && (box[e] != 0 || box[e3 + e] != 0 || box[2 * e3 + e] != 0);
-            int q[3] = {o[0] + e % edge, o[1] + (e / edge) % edge, o[2] + e / (edge * edge)};
             plain[j] = plain_ok;
-            for (int k = 0; k < kBoxNb; k++)
-                if (k < n_nb && in_box_axis(P, 0, q[0], nb_o[k][0]) && in_box_axis(P, 1, q[1], nb_o[k][1]) &&
-                    in_box_axis(P, 2, q[2], nb_o[k][2]))
-                    plain[j] = false;
-            for (int a = 0; a < 3; a++) {
-                const int n = axis_n(P, a);
-                if (P.periodic[a]) q[a] = wrap_axis(q[a], n);
-                else if (q[a] < 0 || q[a] >= n) on[j] = false;
+            int q[3] = {0, 0, 0};
+            if (on[j]) {                // a slab fills few of a round's places
+                const int ey = e / edge, ez = ey / edge;
+                q[0] = o[0] + e - ey * edge; q[1] = o[1] + ey - ez * edge; q[2] = o[2] + s0 + ez;
+#pragma unroll 1
+                for (int k = 0; k < n_nb; k++)
+                    if (in_box_axis(P, 0, q[0], nb_o[k][0]) && in_box_axis(P, 1, q[1], nb_o[k][1]) &&
+                        in_box_axis(P, 2, q[2], nb_o[k][2]))
+                        plain[j] = false;
+                for (int a = 0; a < 3; a++) {
+                    const int n = axis_n(P, a);
+                    if (P.periodic[a]) q[a] = wrap_axis(q[a], n);
+                    else if (q[a] < 0 || q[a] >= n) on[j] = false;
+                }
             }
             kk[j] = on[j] ? ((size_t)q[2] * P.ny + q[1]) * P.nx + q[0] : 0;
             rec[j] = on[j] ? fl.stage[kk[j]] : StageRec<float>{1.f, 0.f, 0.f, 0.f};

@@ -1,6 +1,8 @@
 // Launch sequence of the immersed boundary stage (particles FP64; fluid-side
 // fields in the lattice's compute type). The tile macroscopics kernel, which
 // reads the populations, is launched from the per-precision kernel files.
+#include <algorithm>
+
 #include "ibm_kernels.h"
 
 namespace vlbm {
@@ -17,6 +19,15 @@ static int spread(const IbmParams& P, const IbmFluid<T>& fl, hipStream_t st) {
     return 0;
 }
 
+// z-slabs of a sphere's box: as many as keep one workgroup per CU (its 1024
+// threads and 91 registers fill the CU), at most 8, as every slab reads all nodes
+// of the sphere. 48 spheres of radius 8 and 804 nodes, us a launch: 1 slab 51,
+// 5 slabs 29, 8 slabs (a second round of workgroups) 33.
+static int box_slabs(int n_spheres, int edge) {
+    const int s = 256 / (n_spheres > 0 ? n_spheres : 1);
+    return s < 1 ? 1 : std::min({s, 8, edge});
+}
+
 template <>
 int spread<float>(const IbmParams& P, const IbmFluid<float>& fl, hipStream_t st) {
     if (P.box_edge <= 0) {
@@ -24,7 +35,9 @@ int spread<float>(const IbmParams& P, const IbmFluid<float>& fl, hipStream_t st)
                            st, P, fl);
         return 0;
     }
-    const size_t lds = 3 * sizeof(int) * (size_t)P.box_edge * P.box_edge * P.box_edge;
+    const int slabs = box_slabs(P.n_spheres, P.box_edge);
+    const size_t planes = (size_t)((P.box_edge + slabs - 1) / slabs);
+    const size_t lds = 3 * sizeof(int) * planes * P.box_edge * P.box_edge;
     static size_t lds_set = 0;
     if (lds > lds_set) {
         if (hipFuncSetAttribute((const void*)k_ibm_spread_box, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -32,7 +45,7 @@ int spread<float>(const IbmParams& P, const IbmFluid<float>& fl, hipStream_t st)
             return -1;
         lds_set = lds;
     }
-    hipLaunchKernelGGL(k_ibm_spread_box, dim3((uint32_t)P.n_spheres), dim3(kSphereBlock), lds, st, P, fl);
+    hipLaunchKernelGGL(k_ibm_spread_box, dim3((uint32_t)P.n_spheres, (uint32_t)slabs), dim3(kSphereBlock), lds, st, P, fl);
     return 0;
 }
 
