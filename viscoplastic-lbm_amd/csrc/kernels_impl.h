@@ -787,11 +787,10 @@ __device__ __forceinline__ uint32_t tile_of(const Params<T>& p, int x, int y, in
     return tile_index(x, y, z, p.tiles_x, p.tiles_y);
 }
 
-// 16-bit storage keeps the sums and products of the collision in one order:
-// stochastic rounding turns a change in the last bit of a float into a whole
-// step of the stored 16-bit value.
-template <typename S> constexpr bool kSequential = sizeof(S) == 2;
-
+// Steps on populations are bound by memory and evaluate sums and products
+// population by population. The pairwise forms of the coefficient steps differ
+// in the last bit, which stochastic rounding to 16 bits turns into whole steps of
+// the stored value.
 // omega_old: power-law state of the node (ignored otherwise).
 template <int Q, int RHEO, bool SEQ, typename T>
 __device__ __forceinline__ Moments<Q, RHEO, T> moments(const T* g, const Params<T>& p, T omega_old,
@@ -913,17 +912,9 @@ __device__ __forceinline__ void coeffs_collide(T* c, const Moments<Q, RHEO, T>& 
     c[9] = r9 * m.uy * m.uz + b9 * (m.uy * F.z + m.uz * F.y) + a2 * m.pyz;
 }
 
-// The regularized collision as populations.
+// The same collision population by population.
 template <int Q, int RHEO, typename T>
 __device__ __forceinline__ void collide(T* g, const Moments<Q, RHEO, T>& m, const Force<T>& F) {
-    T c[kCoef];
-    coeffs_collide<Q, RHEO, T>(c, m, F);
-    expand<Q, T>(c, g);
-}
-
-// The same collision population by population (kSequential).
-template <int Q, int RHEO, typename T>
-__device__ __forceinline__ void collide_seq(T* g, const Moments<Q, RHEO, T>& m, const Force<T>& F) {
     const T om = m.omega;
     const T a = (T)4.5 * ((T)1 - om);
     const T b = (T)1 - (T)0.5 * om;
@@ -993,13 +984,13 @@ __device__ __forceinline__ Force<T> node_force(const Params<T>& p, const Node<T>
 // Moments, apparent omega, saved macroscopics and collision of one node whose
 // post-stream, post-BC deviations are g; the post-collision state goes to
 // dst in representation OUT. om_old: the power law's omega of the node.
-template <int Q, typename S, int RHEO, int OUT>
+template <int Q, typename S, int RHEO, int IN, int OUT>
 __device__ __forceinline__ void collide_store(const Params<typename ComputeOf<S>::type>& p, uint32_t idx,
                                               typename ComputeOf<S>::type* g,
                                               const Force<typename ComputeOf<S>::type>& F,
                                               typename ComputeOf<S>::type om_old) {
     using T = typename ComputeOf<S>::type;
-    const Moments<Q, RHEO, T> m = moments<Q, RHEO, kSequential<S>>(g, p, om_old, F);
+    const Moments<Q, RHEO, T> m = moments<Q, RHEO, IN == kRepPop>(g, p, om_old, F);
     if (RHEO == 2) p.omega_state[idx] = m.omega;
     // LES_EXPORT_VISC_TURBULENT: every step, as the reference (lbm.cu:237-239)
     if (RHEO == 0 && p.visc_turb) p.visc_turb[idx] = m.tau_t / (T)3;
@@ -1016,7 +1007,6 @@ __device__ __forceinline__ void collide_store(const Params<typename ComputeOf<S>
         return;
     }
     if (p.bgk) collide_bgk<Q, RHEO, T>(g, m, F);
-    else if constexpr (kSequential<S>) collide_seq<Q, RHEO, T>(g, m, F);
     else collide<Q, RHEO, T>(g, m, F);
     if constexpr (sizeof(S) == 2) {
         if (p.sr) {
@@ -1063,7 +1053,7 @@ __device__ __forceinline__ void step_node(const Params<typename ComputeOf<S>::ty
         gather<Q, T>(g, pc);
         if (w_scheme(word) != kNull) apply_bc<Q, T, MASK>(g, p, nd, word, pc);
     }
-    collide_store<Q, S, RHEO, OUT>(p, idx, g, node_force<IBM>(p, nd), RHEO == 2 ? p.omega_state[idx] : (T)0);
+    collide_store<Q, S, RHEO, IN, OUT>(p, idx, g, node_force<IBM>(p, nd), RHEO == 2 ? p.omega_state[idx] : (T)0);
 }
 
 // One pulled step of a population node (gather_rows); every thread of the
@@ -1111,7 +1101,7 @@ __device__ __forceinline__ void step_node_rows(const Params<typename ComputeOf<S
         if (!in || !w_used(word)) return;
         if (w_scheme(word) != kNull) apply_bc<Q, T, MASK>(g, p, nd, word, GlobalPC<Q, S, T, kRepPop>{p, nd});
     }
-    collide_store<Q, S, RHEO, OUT>(p, idx, g, node_force<IBM>(p, nd), RHEO == 2 ? p.omega_state[idx] : (T)0);
+    collide_store<Q, S, RHEO, kRepPop, OUT>(p, idx, g, node_force<IBM>(p, nd), RHEO == 2 ? p.omega_state[idx] : (T)0);
 }
 
 // One time step over the lattice, one node per thread; ROWS: pull through
@@ -1204,7 +1194,7 @@ __global__ __launch_bounds__(kBlock) void k_aux(const Params<typename ComputeOf<
     }
     if (!w_used(word)) return;
     const T om_old = (RHEO == 2) ? p.omega_state[idx] : (T)0;
-    const Moments<Q, RHEO, T> m = moments<Q, RHEO, kSequential<S>>(g, p, om_old, const_force(p));
+    const Moments<Q, RHEO, T> m = moments<Q, RHEO, IN == kRepPop>(g, p, om_old, const_force(p));
     p.m_rho[idx] = m.rho; p.m_ux[idx] = m.ux; p.m_uy[idx] = m.uy; p.m_uz[idx] = m.uz;
     if (RHEO != 0) p.m_omega[idx] = m.omega;
 }
@@ -1237,7 +1227,7 @@ __global__ __launch_bounds__(kBlock) void k_ibm_macr(const Params<typename Compu
             gather<Q, T>(g, pc);
             if (w_scheme(word) != kNull) apply_bc<Q, T, MASK>(g, p, nd, word, pc);
         }
-        const Moments<Q, 0, T> m = moments<Q, 0, kSequential<S>>(g, p, (T)0, const_force(p));
+        const Moments<Q, 0, T> m = moments<Q, 0, IN == kRepPop>(g, p, (T)0, const_force(p));
         p.ibm_stage[idx] = StageRec<T>{m.rho, m.ux, m.uy, m.uz};
         ffx[idx] = p.fx; ffy[idx] = p.fy; ffz[idx] = p.fz;
     }

@@ -257,7 +257,7 @@ __global__ __launch_bounds__((TileShape<T, Q>::NT), (TileShape<T, Q>::MIN_WAVES)
             if (w_used(word)) {
                 if (w_scheme(word) != kNull)
                     apply_bc<Q, T, MASK>(low, p, nd, word, ColumnPC<Q, T>{below, wall_a, &wall_of, {p, nd}});
-                collide_store<Q, T, RHEO, kRepMom>(p, nd.idx, low, IBM ? F : const_force(p), om);
+                collide_store<Q, T, RHEO, kRepMom, kRepMom>(p, nd.idx, low, IBM ? F : const_force(p), om);
             }
         }
         word = word_next;
