@@ -9,12 +9,14 @@
 #include <cstdlib>
 #include <cstring>
 #include <thread>
+#include <vector>
 
 namespace vlbm {
 namespace detail {
 namespace {
 
 constexpr int kThreads = 4;
+constexpr size_t kStagedBytes = size_t(16) << 20;
 
 // CPUs this process may run on.
 int cpus() {
@@ -41,6 +43,15 @@ void run_workers(int workers, F&& fn) {
     for (int t = 0; t < started; t++) threads[t].join();
 }
 
+// Writes to every page of [p, p + bytes) without changing it: another thread
+// may be storing the values already.
+void fault_in(char* p, size_t bytes) {
+    for (size_t k = 0; k < bytes; k += 4096) {
+        char c = __atomic_load_n(p + k, __ATOMIC_RELAXED);
+        (void)__atomic_compare_exchange_n(p + k, &c, c, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED);
+    }
+}
+
 }  // namespace
 
 void widen(double* out, const void* in, size_t n, int value_bytes) {
@@ -55,8 +66,10 @@ void widen(double* out, const void* in, size_t n, int value_bytes) {
 hipError_t HostCopy::reserve(int slots, size_t bytes) {
     slots = std::min(slots, kSlots);
     if (bytes > slot_bytes_) {
+        // by powers of two: an owner of fields of many sizes grows a few times only
         release();
-        slot_bytes_ = bytes;
+        slot_bytes_ = size_t(64) << 10;
+        while (slot_bytes_ < bytes) slot_bytes_ *= 2;
     }
     for (; slots_ < slots; slots_++) {
         void* p = nullptr;
@@ -89,14 +102,28 @@ void HostCopy::release() {
     slot_bytes_ = 0;
 }
 
+// Field by field through the runtime's own staging.
+hipError_t HostCopy::fetch_small(hipStream_t stream, const FieldCopy* fields, int count, size_t n, int value_bytes, bool raw) {
+    const bool convert = !raw && value_bytes == 4;
+    for (int f = 0; f < count; f++) {
+        std::vector<float> tmp(convert ? n : 0);
+        hipError_t e = hipMemcpyAsync(convert ? (void*)tmp.data() : fields[f].out, fields[f].dev, n * (size_t)value_bytes,
+                                      hipMemcpyDeviceToHost, stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(stream);
+        if (e != hipSuccess) return e;
+        if (convert) widen((double*)fields[f].out, tmp.data(), n, 4);
+    }
+    return hipSuccess;
+}
+
 hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fields, int count, size_t n,
                            int value_bytes, bool raw) {
-    std::lock_guard<std::mutex> lock(mu_);
     const size_t vb = (size_t)value_bytes, total = n * (size_t)count * vb;
-    // slots of 2 MB with threads, of 512 KB without (the first copy, which nothing overlaps, is shorter)
-    const bool threads = total >= (size_t(16) << 20);
-    const size_t per = std::min(n, (threads ? kSlotBytes : kSlotBytes / 4) / vb);        // values of a chunk
-    const size_t per_field = per ? (n + per - 1) / per : 0, chunks = per_field * (size_t)count;
+    if (total < kStagedBytes) return fetch_small(stream, fields, count, n, value_bytes, raw);
+    std::lock_guard<std::mutex> lock(mu_);
+    // equal chunks of a field, none larger than a slot
+    const size_t per_field = (n * vb + kSlotBytes - 1) / kSlotBytes, chunks = per_field * (size_t)count;
+    const size_t per = per_field ? (n + per_field - 1) / per_field : 0;                  // values of a chunk
     if (!chunks) return hipSuccess;
     hipError_t e = reserve((int)std::min<size_t>(chunks, kSlots), per * vb);
     if (e != hipSuccess) return e;
@@ -120,16 +147,6 @@ hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fiel
         else widen((double*)c.out, slot_[s], c.n, value_bytes);
         return hipSuccess;
     };
-    if (!threads) {
-        const size_t ahead = (size_t)slots_;
-        for (size_t i = 0; i < std::min(ahead, chunks) && e == hipSuccess; i++) e = enqueue(i, (int)i);
-        for (size_t i = 0; i < chunks && e == hipSuccess; i++) {
-            e = finish(i, (int)(i % ahead));
-            if (e == hipSuccess && i + ahead < chunks) e = enqueue(i + ahead, (int)(i % ahead));
-        }
-        if (e != hipSuccess) (void)hipStreamSynchronize(stream);      // no copy into a slot outlives the call
-        return e;
-    }
     std::atomic<size_t> touch{0}, next{0};
     std::atomic<int> error{(int)hipSuccess};
     std::atomic<bool> ready{false};
@@ -149,7 +166,7 @@ hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fiel
             // the pages of the destination, while the stream computes
             for (size_t i; !ready && (i = touch++) < chunks;) {
                 const Chunk c = chunk(i);
-                for (size_t k = 0; k < c.n * ob && !ready; k += 4096) *(volatile char*)(c.out + k) = 0;
+                fault_in(c.out, c.n * ob);
             }
             std::unique_lock<std::mutex> g(m);
             cv.wait(g, [&] { return ready.load(); });

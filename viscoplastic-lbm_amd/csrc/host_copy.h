@@ -2,16 +2,15 @@
 //
 // What bounds it is the host: the link carries 55 GB/s, while one thread that
 // lets the runtime stage a pageable copy into a fresh temporary and then
-// converts it writes every page three times and faults it in twice (four
-// fields of a 256^3 float lattice: 107 ms, of which the link needs 5). Here the
-// copies go into page-locked slots and are converted from there into place. From
-// 16 MB on, 4 threads each take the next chunk, so the page faults and
-// conversions of different chunks overlap, and while the stream still computes
-// they fault in the destination: 17 ms for those fields after an idle stream (8
-// threads 14, 2 27, 1 45), about 8 behind 200 steps. Below, one thread with all
-// slots in flight: threads gain little there and get in the way of a caller's own
-// pool (four fields of 0.6 million nodes between torch operations: 2 to 6 ms with
-// 4 threads, 1.4 with one).
+// converts it writes every page three times and faults it in twice (the four
+// fields of a 256^3 float lattice: 107 ms, of which the link needs 5). From 16 MB
+// on, 4 threads each take the next chunk, copy it into a page-locked slot of their
+// own and convert it into place, so the link, the page faults and the conversion of
+// different chunks overlap; while the stream still computes they fault in the
+// destination. Those fields then take 17 ms after an idle stream (8 threads 14,
+// 2 27, 1 45), about 8 behind 200 steps. Below 16 MB the runtime's staging is the
+// faster one (0.6 million float nodes 1.4 ms; one thread over slots 1.2 to 2.0, four
+// 2 to 6 between the caller's own parallel operations).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -26,7 +25,7 @@ struct FieldCopy {
     void* out;            // on the host: n doubles, or n values as they are on the device
 };
 
-// Page-locked staging of one owner (a lattice handle, a batch): at most 8
+// Page-locked staging of one owner (a lattice handle, a batch): at most 4
 // slots of 2 MB, allocated by the first download that needs them and freed
 // with the owner. Downloads of one owner from several threads take turns.
 class HostCopy {
@@ -42,7 +41,8 @@ public:
     void release();
 
 private:
-    static constexpr int kSlots = 8;
+    static hipError_t fetch_small(hipStream_t stream, const FieldCopy* fields, int count, size_t n, int value_bytes, bool raw);
+    static constexpr int kSlots = 4;
     static constexpr size_t kSlotBytes = size_t(2) << 20;
     hipError_t reserve(int slots, size_t bytes);
     std::mutex mu_;

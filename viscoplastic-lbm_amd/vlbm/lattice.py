@@ -150,8 +150,8 @@ class Lattice:
         check(lib.vlbm_compute_macroscopics(self._h))
 
     def macroscopics(self, omega: bool = False) -> dict:
-        out = {k: np.empty(self.shape) for k in ("rho", "ux", "uy", "uz")}
-        om = np.empty(self.shape) if omega else None
+        out = {k: np.zeros(self.shape) for k in ("rho", "ux", "uy", "uz")}
+        om = np.zeros(self.shape) if omega else None
         check(lib.vlbm_macroscopics(self._h, _ptr(out["rho"]), _ptr(out["ux"]), _ptr(out["uy"]),
                                     _ptr(out["uz"]), _ptr(om)))
         if omega:

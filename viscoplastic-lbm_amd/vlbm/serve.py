@@ -126,7 +126,7 @@ class Batch:
                 "t_submit": i.t_submit, "t_start": i.t_start, "t_end": i.t_end, "bytes": i.bytes}
 
     def result(self, jid: int, shape) -> Dict[str, np.ndarray]:
-        out = {k: np.empty(shape) for k in ("rho", "ux", "uy", "uz")}
+        out = {k: np.zeros(shape) for k in ("rho", "ux", "uy", "uz")}
         dp = C.POINTER(C.c_double)
         check(lib.vlbm_batch_job_result(self._h, int(jid), *[out[k].ctypes.data_as(dp) for k in ("rho", "ux", "uy", "uz")]))
         return out
