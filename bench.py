@@ -268,7 +268,7 @@ def main():
             "tau": 0.8, "yield_stress": 1e-5, "u_inlet": 0.01,
             "layout": layout,
             "storage": ("fp32 regularized-state coefficients (10 per node), two lattices, pull streaming through "
-                        "an LDS plane ring" if layout == "moments" else
+                        "an LDS exchange" if layout == "moments" else
                         "fp32 deviations f_i - w_i, two lattices, pull streaming"),
             "device_settle": f"{settled_steps} step launches ({args.settle:g} s) on a separate 256^3 lattice "
                              "before the warm-up",
