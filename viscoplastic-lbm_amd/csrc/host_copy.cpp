@@ -16,7 +16,7 @@ namespace detail {
 namespace {
 
 constexpr int kThreads = 4;
-constexpr size_t kStagedBytes = size_t(16) << 20;
+constexpr size_t kStagedBytes = size_t(16) << 20, kThreadBytes = size_t(128) << 20;
 
 // CPUs this process may run on.
 int cpus() {
@@ -147,6 +147,18 @@ hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fiel
         else widen((double*)c.out, slot_[s], c.n, value_bytes);
         return hipSuccess;
     };
+    if (total < kThreadBytes) {
+        // all slots in flight; the destination is faulted in while the stream computes
+        const size_t ahead = (size_t)slots_;
+        for (size_t i = 0; i < std::min(ahead, chunks) && e == hipSuccess; i++) e = enqueue(i, (int)i);
+        for (size_t i = 0; i < chunks && e == hipSuccess; i++) fault_in(chunk(i).out, chunk(i).n * ob);
+        for (size_t i = 0; i < chunks && e == hipSuccess; i++) {
+            e = finish(i, (int)(i % ahead));
+            if (e == hipSuccess && i + ahead < chunks) e = enqueue(i + ahead, (int)(i % ahead));
+        }
+        if (e != hipSuccess) (void)hipStreamSynchronize(stream);      // no copy into a slot outlives the call
+        return e;
+    }
     std::atomic<size_t> touch{0}, next{0};
     std::atomic<int> error{(int)hipSuccess};
     std::atomic<bool> ready{false};

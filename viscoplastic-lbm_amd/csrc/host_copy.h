@@ -4,13 +4,14 @@
 // lets the runtime stage a pageable copy into a fresh temporary and then
 // converts it writes every page three times and faults it in twice (the four
 // fields of a 256^3 float lattice: 107 ms, of which the link needs 5). From 16 MB
-// on, 4 threads each take the next chunk, copy it into a page-locked slot of their
-// own and convert it into place, so the link, the page faults and the conversion of
-// different chunks overlap; while the stream still computes they fault in the
-// destination. Those fields then take 17 ms after an idle stream (8 threads 14,
-// 2 27, 1 45), about 8 behind 200 steps. Below 16 MB the runtime's staging is the
-// faster one (0.6 million float nodes 1.4 ms; one thread over slots 1.2 to 2.0, four
-// 2 to 6 between the caller's own parallel operations).
+// on, copies go into page-locked slots, all in flight, and are converted from there
+// into place; the destination is faulted in while the stream still computes, which
+// is half of the time. From 128 MB on 4 threads share the chunks: those fields then
+// take 17 ms after an idle stream (8 threads 14, 2 27, 1 45), about 8 behind 200
+// steps. Smaller downloads stay on one thread: with threads a pass of 9 ms and 28 MB
+// took 11.4 or 23 ms, run by run, beside a caller's own spinning pool. Below 16 MB
+// the runtime's staging is the faster one (0.6 million float nodes 1.4 ms, slots 1.2
+// to 2.0).
 #pragma once
 #include <hip/hip_runtime.h>
 

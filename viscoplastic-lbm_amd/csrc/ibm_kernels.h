@@ -16,7 +16,7 @@
 //             forces / moments (fixed-order tree); sphere sums and velocity
 //             update; spreading of the node forces straight into u (F / 2 rho)
 //             and the force field, through an LDS box around each sphere for
-//             FP32 fluids (one workgroup per sphere)
+//             FP32 fluids (one workgroup per z-slab of a box)
 //   move      sphere and node movement
 // Everything outside the flagged tiles is left alone: the reference's full-
 // lattice passes (gpuUpdateMacrIBM, gpuEulerSumIBMAuxsReset over the bordered
@@ -924,14 +924,30 @@ __global__ __launch_bounds__(kInterpBlock) void k_ibm_interp(IbmParams P, IbmFlu
     }
 }
 
-// chunk sums -> sphere force and torque, chunks in order; velocity update
-__global__ __launch_bounds__(kIbmBlock) void k_ibm_add_chunks(IbmParams P) {
-    const int s = blockIdx.x * kIbmBlock + threadIdx.x;
-    if (s >= P.n_spheres) return;
-    IbmSphere& c = P.sph[s];
+// Value of lane j (the same j in every lane).
+__device__ __forceinline__ double lane_value(double v, int j) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), j),
+                            __builtin_amdgcn_readlane(__double2loint(v), j));
+}
+
+// chunk sums -> sphere force and torque, chunks in order; velocity update. One
+// wave per sphere: the lanes load a chunk's sums each, and the sums are added in
+// chunk order from the lanes' registers. Latency bound: one thread per sphere took
+// a memory latency per chunk (13 chunks, 8.6 us).
+__global__ __launch_bounds__(64) void k_ibm_add_chunks(IbmParams P) {
+    const int s = (int)blockIdx.x, lane = (int)threadIdx.x;
+    const int k0 = P.chunk0[s], k1 = P.chunk0[s + 1];
     double t[6] = {0, 0, 0, 0, 0, 0};
-    for (int k = P.chunk0[s]; k < P.chunk0[s + 1]; k++)
-        for (int a = 0; a < 6; a++) t[a] += P.chunk_sums[6 * k + a];
+    for (int b = k0; b < k1; b += 64) {
+        double v[6] = {0, 0, 0, 0, 0, 0};
+        if (b + lane < k1)
+            for (int a = 0; a < 6; a++) v[a] = P.chunk_sums[6 * (b + lane) + a];
+        const int n = min(64, k1 - b);
+        for (int j = 0; j < n; j++)
+            for (int a = 0; a < 6; a++) t[a] += lane_value(v[a], j);
+    }
+    if (lane != 0) return;
+    IbmSphere& c = P.sph[s];
     for (int a = 0; a < 3; a++) { c.f[a] += t[a]; c.M[a] += t[3 + a]; }
     sphere_velocity(P, s);
 }

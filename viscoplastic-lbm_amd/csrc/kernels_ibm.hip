@@ -70,7 +70,7 @@ static int stage_part(const IbmParams& P, const IbmFluid<T>& fl, int part, hipSt
     case kIbmIteration:
         if (nn) {
             hipLaunchKernelGGL((k_ibm_interp<T>), dim3(xcd_chunk_grid(P.n_chunks)), dim3(kInterpBlock), 0, st, P, fl);
-            hipLaunchKernelGGL(k_ibm_add_chunks, blocks_for(ns), blk, 0, st, P);   // with the velocity update
+            hipLaunchKernelGGL(k_ibm_add_chunks, dim3(ns), dim3(64), 0, st, P);   // with the velocity update
         } else if (ns) {
             hipLaunchKernelGGL(k_ibm_velocity, blocks_for(ns), blk, 0, st, P);
         }
