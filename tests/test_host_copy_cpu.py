@@ -1,0 +1,24 @@
+"""Staging of the field downloads (csrc/host_copy.cpp) on the CPU: the file is
+compiled with g++ over a model of the HIP runtime (host_stub/), which has two
+devices and runs a stream only when somebody waits for it."""
+import subprocess
+from pathlib import Path
+
+import pytest
+
+HERE = Path(__file__).resolve().parent
+CSRC = HERE.parent / "viscoplastic-lbm_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("host_copy") / "check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-pthread", "-I", str(HERE / "host_stub"), "-I", str(CSRC),
+                    str(HERE / "host_stub" / "host_copy_check.cpp"), str(CSRC / "host_copy.cpp"), "-o", str(exe)], check=True)
+    return exe
+
+
+@pytest.mark.parametrize("name", ["other_device"])
+def test_download(program, name):
+    res = subprocess.run([str(program), name], capture_output=True, text=True, timeout=100)
+    assert res.returncode == 0, res.stdout + res.stderr

@@ -11,6 +11,8 @@
 #include <thread>
 #include <vector>
 
+#include "device_scope.h"
+
 namespace vlbm {
 namespace detail {
 namespace {
@@ -121,6 +123,8 @@ hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fiel
     const size_t vb = (size_t)value_bytes, total = n * (size_t)count * vb;
     if (total < kStagedBytes) return fetch_small(stream, fields, count, n, value_bytes, raw);
     std::lock_guard<std::mutex> lock(mu_);
+    const DeviceScope scope(device);         // the caller's current device may be another one
+    if (!scope.ok) return hipErrorInvalidDevice;
     // equal chunks of a field, none larger than a slot
     const size_t per_field = (n * vb + kSlotBytes - 1) / kSlotBytes, chunks = per_field * (size_t)count;
     const size_t per = per_field ? (n + per_field - 1) / per_field : 0;                  // values of a chunk

@@ -14,6 +14,7 @@
 
 #include "../../include/vlbm.h"
 #include "ctx.h"
+#include "device_scope.h"
 #include "lattice.h"
 
 using namespace vlbm;
@@ -47,19 +48,6 @@ int scratch_on(int device, double** out) {
     *out = g_scratch_ptr[device];
     return VLBM_OK;
 }
-
-// Makes the handle's device current for the call and restores the caller's.
-struct DeviceScope {
-    int prev = -1;
-    bool ok = false;
-    explicit DeviceScope(int device) {
-        if (hipGetDevice(&prev) != hipSuccess) return;
-        ok = prev == device || hipSetDevice(device) == hipSuccess;
-    }
-    ~DeviceScope() {
-        if (ok && prev >= 0) (void)hipSetDevice(prev);
-    }
-};
 
 // One chunk of the aux kernel (kAuxMaterialize to doubles, or kAuxGhost)
 // into the scratch: Q planes of `count` values.
