@@ -53,10 +53,33 @@ int other_device() {
     return 0;
 }
 
+// A download into fresh memory takes one page fault a page: the first access
+// of each page is a write.
+int page_faults() {
+    const size_t n = kOneThread, bytes = 4 * n * sizeof(double);
+    char* out = (char*)mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+    if (out == MAP_FAILED) return fail("set-up");
+    (void)madvise(out, bytes, MADV_NOHUGEPAGE);
+    stub::Stream s{0};
+    Fields a(n);
+    HostCopy owner;
+    if (owner.fetch(0, &s, a.list.data(), 4, n, 4) != hipSuccess) return fail("download");      // touches the slots
+    for (int f = 0; f < 4; f++) a.list[f].out = out + f * n * sizeof(double);
+    struct rusage before, after;
+    getrusage(RUSAGE_SELF, &before);
+    if (owner.fetch(0, &s, a.list.data(), 4, n, 4) != hipSuccess) return fail("download");
+    getrusage(RUSAGE_SELF, &after);
+    const double faults = (double)(after.ru_minflt - before.ru_minflt), pages = bytes / 4096.0;
+    std::printf("%.0f faults, %.0f pages\n", faults, pages);
+    if (std::memcmp(out, a.out.data(), bytes) != 0) return fail("wrong values");
+    return faults <= 1.1 * pages ? 0 : fail("more than one fault a page");
+}
+
 }  // namespace
 
 int main(int, char** argv) {
     const std::string name = argv[1];
     if (name == "other_device") return other_device();
+    if (name == "page_faults") return page_faults();
     return fail("unknown check");
 }

@@ -46,11 +46,15 @@ void run_workers(int workers, F&& fn) {
 }
 
 // Writes to every page of [p, p + bytes) without changing it: another thread
-// may be storing the values already.
+// may be storing the values already. The compare-exchange is the first access of
+// the page and writes on x86 whatever it finds; a load before it would fault the
+// page in for reading first, a second fault a page (30 MB of float fields into
+// fresh 4 KB pages after an idle stream: 15.0 ms with the load, 9.5 without,
+// 11.9 through the runtime's own staging).
 void fault_in(char* p, size_t bytes) {
     for (size_t k = 0; k < bytes; k += 4096) {
-        char c = __atomic_load_n(p + k, __ATOMIC_RELAXED);
-        (void)__atomic_compare_exchange_n(p + k, &c, c, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED);
+        char zero = 0;
+        (void)__atomic_compare_exchange_n(p + k, &zero, (char)0, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED);
     }
 }
 
