@@ -75,11 +75,26 @@ int page_faults() {
     return faults <= 1.1 * pages ? 0 : fail("more than one fault a page");
 }
 
+// Neither page-locked memory nor events to be had: the runtime's staging serves.
+int refused() {
+    for (int k = 0; k < 3; k++) {
+        stub::refuse_host_malloc = k != 1;
+        stub::refuse_events = k > 0;
+        stub::Stream s{0};
+        Fields a(kOneThread);
+        HostCopy owner;
+        if (owner.fetch(0, &s, a.list.data(), 4, a.n, 4) != hipSuccess) return fail("download refused");
+        if (!a.right()) return fail("wrong values");
+    }
+    return stub::host_live == 0 && stub::events_live == 0 ? 0 : fail("slots that are not page-locked were kept");
+}
+
 }  // namespace
 
 int main(int, char** argv) {
     const std::string name = argv[1];
     if (name == "other_device") return other_device();
     if (name == "page_faults") return page_faults();
+    if (name == "refused") return refused();
     return fail("unknown check");
 }

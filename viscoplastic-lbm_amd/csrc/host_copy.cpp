@@ -133,8 +133,9 @@ hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fiel
     const size_t per_field = (n * vb + kSlotBytes - 1) / kSlotBytes, chunks = per_field * (size_t)count;
     const size_t per = per_field ? (n + per_field - 1) / per_field : 0;                  // values of a chunk
     if (!chunks) return hipSuccess;
-    hipError_t e = reserve((int)std::min<size_t>(chunks, kSlots), per * vb);
-    if (e != hipSuccess) return e;
+    hipError_t e = hipSuccess;
+    if (reserve((int)std::min<size_t>(chunks, kSlots), per * vb) != hipSuccess)
+        return fetch_small(stream, fields, count, n, value_bytes, raw);
     struct Chunk { const char* dev; char* out; size_t n; };
     const size_t ob = raw ? vb : sizeof(double);
     auto chunk = [&](size_t i) {
