@@ -2,8 +2,10 @@
 #include <sys/mman.h>
 #include <sys/resource.h>
 
+#include <atomic>
 #include <cstdio>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "host_copy.h"
@@ -75,6 +77,36 @@ int page_faults() {
     return faults <= 1.1 * pages ? 0 : fail("more than one fault a page");
 }
 
+// Lattices opened one after the other, as a parameter study does: only the
+// first download in the process pays for page-locked memory. Downloads at once
+// each have slots of their own; what is kept afterwards is bounded, per device.
+int new_owners() {
+    for (int k = 0; k < 5; k++) {
+        stub::Stream s{k & 1};
+        Fields a(k < 3 ? kOneThread : kThreads);
+        HostCopy owner;
+        if (owner.fetch(k & 1, &s, a.list.data(), 4, a.n, 4) != hipSuccess) return fail("download");
+        if (!a.right()) return fail("wrong values");
+    }
+    std::printf("%d page-locked blocks for two devices\n", stub::host_allocs.load());
+    if (stub::host_allocs > 8) return fail("new lattices page-lock memory of their own");
+    std::atomic<int> wrong{0};
+    std::vector<std::thread> threads;
+    for (int k = 0; k < 6; k++)
+        threads.emplace_back([&wrong, k] {
+            for (int r = 0; r < 3; r++) {
+                stub::Stream s{k & 1};
+                Fields a(k < 5 ? kOneThread + k : kThreads);
+                HostCopy owner;
+                if (owner.fetch(k & 1, &s, a.list.data(), 4, a.n, 4) != hipSuccess || !a.right()) wrong++;
+            }
+        });
+    for (auto& t : threads) t.join();
+    if (wrong) return fail("wrong values from downloads at once");
+    std::printf("%d blocks and %d events kept\n", stub::host_live.load(), stub::events_live.load());
+    return stub::host_live <= 8 && stub::events_live <= 8 ? 0 : fail("more kept than 4 slots a device");
+}
+
 // Neither page-locked memory nor events to be had: the runtime's staging serves.
 int refused() {
     for (int k = 0; k < 3; k++) {
@@ -95,6 +127,7 @@ int main(int, char** argv) {
     const std::string name = argv[1];
     if (name == "other_device") return other_device();
     if (name == "page_faults") return page_faults();
+    if (name == "new_owners") return new_owners();
     if (name == "refused") return refused();
     return fail("unknown check");
 }

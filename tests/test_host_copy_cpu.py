@@ -18,7 +18,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("name", ["other_device", "page_faults", "refused"])
+@pytest.mark.parametrize("name", ["other_device", "page_faults", "refused", "new_owners"])
 def test_download(program, name):
     res = subprocess.run([str(program), name], capture_output=True, text=True, timeout=100)
     assert res.returncode == 0, res.stdout + res.stderr

@@ -89,7 +89,6 @@ struct vlbm_batch {
     std::map<std::string, std::array<int, 3>> shapes;   // launch shapes chosen in this batch, by key
     std::multimap<size_t, std::unique_ptr<char[]>> spare;   // released result buffers by size
     size_t spare_bytes = 0;
-    HostCopy host_copy;                        // staging of the result downloads
     int device = 0;                            // device current at vlbm_batch_create (the stream's device)
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -312,7 +311,7 @@ int retire(vlbm_batch* b, int id, int state) {
     if ((rc = take_result(b, j, 4 * fb))) return rc;
     FieldCopy fields[4];
     for (int f = 0; f < 4; f++) fields[f] = FieldCopy{idle + f * fb, j.res.get() + f * fb};
-    HIP_TRY(b->host_copy.fetch(b->device, b->stream, fields, 4, n, b->tbytes, true));
+    HIP_TRY(HostCopy::fetch(b->device, b->stream, fields, 4, n, b->tbytes, true));
     j.has_result = true;
     j.state = state;
     j.t_end = b->now();

@@ -70,7 +70,6 @@ struct vlbm_ctx {
     int device = 0;           // device current at vlbm_create (the stream's device)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     size_t device_bytes = 0;
-    vlbm::detail::HostCopy host_copy;   // staging of the field downloads
     vlbm::IbmState* ibm = nullptr;   // immersed boundary stage (vlbm_ibm_enable)
     // what the step kernel needs of the IBM stage (null without IBM)
     const uint32_t* tile_flag = nullptr;
@@ -206,7 +205,7 @@ inline int dalloc(vlbm_ctx* h, void** p, size_t bytes) {
 
 // Host copies of fields (compute type) as doubles.
 inline int fetch_fields(vlbm_ctx* h, const FieldCopy* fields, int count) {
-    HIP_TRY(h->host_copy.fetch(h->device, h->stream, fields, count, h->n, h->tbytes));
+    HIP_TRY(HostCopy::fetch(h->device, h->stream, fields, count, h->n, h->tbytes));
     return VLBM_OK;
 }
 

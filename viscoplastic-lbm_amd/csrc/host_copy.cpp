@@ -18,6 +18,8 @@ namespace detail {
 namespace {
 
 constexpr int kThreads = 4;
+constexpr int kSlots = 4;                               // of a download, and kept for a device
+constexpr size_t kSlotBytes = size_t(2) << 20;
 constexpr size_t kStagedBytes = size_t(16) << 20, kThreadBytes = size_t(128) << 20;
 
 // CPUs this process may run on.
@@ -58,6 +60,84 @@ void fault_in(char* p, size_t bytes) {
     }
 }
 
+// One page-locked buffer and the event of the copy into it.
+struct Slot {
+    void* p = nullptr;
+    hipEvent_t event = nullptr;
+    bool pinned = false;
+
+    bool make() {
+        pinned = hipHostMalloc(&p, kSlotBytes, hipHostMallocDefault) == hipSuccess;
+        if (!pinned) {
+            // pageable memory carries the same copy, staged by the runtime
+            (void)hipGetLastError();
+            p = std::malloc(kSlotBytes);
+        }
+        if (p && hipEventCreateWithFlags(&event, hipEventDisableTiming) == hipSuccess) return true;
+        (void)hipGetLastError();
+        event = nullptr;
+        drop();
+        return false;
+    }
+    void drop() {
+        if (event) (void)hipEventDestroy(event);
+        if (pinned) (void)hipHostFree(p);
+        else std::free(p);
+        *this = Slot();
+    }
+};
+
+// Slots of a device that no download holds.
+class SlotPool {
+public:
+    // Up to `want` slots of the current device; fewer when the system has no more.
+    int take(int device, int want, Slot* out) {
+        int got = 0;
+        if (device < kDevices) {
+            std::lock_guard<std::mutex> lock(mu_);
+            while (got < want && count_[device] > 0) out[got++] = idle_[device][--count_[device]];
+        }
+        while (got < want && out[got].make()) got++;
+        return got;
+    }
+    // Slots that no copy is under way into.
+    void give(int device, Slot* slots, int n) {
+        for (int k = 0; k < n; k++) {
+            if (slots[k].pinned && device < kDevices) {
+                std::lock_guard<std::mutex> lock(mu_);
+                if (count_[device] < kSlots) {
+                    idle_[device][count_[device]++] = slots[k];
+                    continue;
+                }
+            }
+            slots[k].drop();
+        }
+    }
+
+private:
+    static constexpr int kDevices = 64;
+    std::mutex mu_;
+    Slot idle_[kDevices][kSlots];
+    int count_[kDevices] = {};
+};
+
+// Never destroyed: at the end of the process the runtime may be gone before it.
+SlotPool& pool() {
+    static SlotPool* p = new SlotPool;
+    return *p;
+}
+
+// The slots of one download.
+struct HeldSlots {
+    const int device;
+    Slot slot[kSlots];
+    const int n;
+    HeldSlots(int device_, int want) : device(device_), n(pool().take(device_, std::min(want, kSlots), slot)) {}
+    HeldSlots(const HeldSlots&) = delete;
+    HeldSlots& operator=(const HeldSlots&) = delete;
+    ~HeldSlots() { pool().give(device, slot, n); }
+};
+
 }  // namespace
 
 void widen(double* out, const void* in, size_t n, int value_bytes) {
@@ -67,45 +147,6 @@ void widen(double* out, const void* in, size_t n, int value_bytes) {
     }
     const float* f = (const float*)in;
     for (size_t k = 0; k < n; k++) out[k] = f[k];
-}
-
-hipError_t HostCopy::reserve(int slots, size_t bytes) {
-    slots = std::min(slots, kSlots);
-    if (bytes > slot_bytes_) {
-        // by powers of two: an owner of fields of many sizes grows a few times only
-        release();
-        slot_bytes_ = size_t(64) << 10;
-        while (slot_bytes_ < bytes) slot_bytes_ *= 2;
-    }
-    for (; slots_ < slots; slots_++) {
-        void* p = nullptr;
-        pinned_[slots_] = hipHostMalloc(&p, slot_bytes_, hipHostMallocDefault) == hipSuccess;
-        if (!pinned_[slots_]) {
-            // pageable memory carries the same copy, staged by the runtime
-            (void)hipGetLastError();
-            p = std::malloc(slot_bytes_);
-            if (!p) break;
-        }
-        if (hipEventCreateWithFlags(&event_[slots_], hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            if (pinned_[slots_]) (void)hipHostFree(p);
-            else std::free(p);
-            break;
-        }
-        slot_[slots_] = p;
-    }
-    return slots_ ? hipSuccess : hipErrorOutOfMemory;
-}
-
-void HostCopy::release() {
-    for (int k = 0; k < slots_; k++) {
-        (void)hipEventDestroy(event_[k]);
-        if (pinned_[k]) (void)hipHostFree(slot_[k]);
-        else std::free(slot_[k]);
-        slot_[k] = nullptr;
-    }
-    slots_ = 0;
-    slot_bytes_ = 0;
 }
 
 // Field by field through the runtime's own staging.
@@ -126,16 +167,15 @@ hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fiel
                            int value_bytes, bool raw) {
     const size_t vb = (size_t)value_bytes, total = n * (size_t)count * vb;
     if (total < kStagedBytes) return fetch_small(stream, fields, count, n, value_bytes, raw);
-    std::lock_guard<std::mutex> lock(mu_);
     const DeviceScope scope(device);         // the caller's current device may be another one
     if (!scope.ok) return hipErrorInvalidDevice;
     // equal chunks of a field, none larger than a slot
     const size_t per_field = (n * vb + kSlotBytes - 1) / kSlotBytes, chunks = per_field * (size_t)count;
     const size_t per = per_field ? (n + per_field - 1) / per_field : 0;                  // values of a chunk
     if (!chunks) return hipSuccess;
+    HeldSlots held(device, (int)std::min<size_t>(chunks, kSlots));
+    if (!held.n) return fetch_small(stream, fields, count, n, value_bytes, raw);
     hipError_t e = hipSuccess;
-    if (reserve((int)std::min<size_t>(chunks, kSlots), per * vb) != hipSuccess)
-        return fetch_small(stream, fields, count, n, value_bytes, raw);
     struct Chunk { const char* dev; char* out; size_t n; };
     const size_t ob = raw ? vb : sizeof(double);
     auto chunk = [&](size_t i) {
@@ -145,20 +185,20 @@ hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fiel
     };
     auto enqueue = [&](size_t i, int s) {
         const Chunk c = chunk(i);
-        const hipError_t ec = hipMemcpyAsync(slot_[s], c.dev, c.n * vb, hipMemcpyDeviceToHost, stream);
-        return ec == hipSuccess ? hipEventRecord(event_[s], stream) : ec;
+        const hipError_t ec = hipMemcpyAsync(held.slot[s].p, c.dev, c.n * vb, hipMemcpyDeviceToHost, stream);
+        return ec == hipSuccess ? hipEventRecord(held.slot[s].event, stream) : ec;
     };
     auto finish = [&](size_t i, int s) {
-        const hipError_t es = hipEventSynchronize(event_[s]);
+        const hipError_t es = hipEventSynchronize(held.slot[s].event);
         if (es != hipSuccess) return es;
         const Chunk c = chunk(i);
-        if (raw) std::memcpy(c.out, slot_[s], c.n * vb);
-        else widen((double*)c.out, slot_[s], c.n, value_bytes);
+        if (raw) std::memcpy(c.out, held.slot[s].p, c.n * vb);
+        else widen((double*)c.out, held.slot[s].p, c.n, value_bytes);
         return hipSuccess;
     };
     if (total < kThreadBytes) {
         // all slots in flight; the destination is faulted in while the stream computes
-        const size_t ahead = (size_t)slots_;
+        const size_t ahead = (size_t)held.n;
         for (size_t i = 0; i < std::min(ahead, chunks) && e == hipSuccess; i++) e = enqueue(i, (int)i);
         for (size_t i = 0; i < chunks && e == hipSuccess; i++) fault_in(chunk(i).out, chunk(i).n * ob);
         for (size_t i = 0; i < chunks && e == hipSuccess; i++) {
@@ -198,7 +238,7 @@ hipError_t HostCopy::fetch(int device, hipStream_t stream, const FieldCopy* fiel
         }
         if (we != hipSuccess) error = (int)we;
     };
-    run_workers(std::min({slots_, kThreads, cpus()}), worker);
+    run_workers(std::min({held.n, kThreads, cpus()}), worker);
     // a copy of a worker that stopped early may still be under way into its slot
     if (error != (int)hipSuccess) (void)hipStreamSynchronize(stream);
     return (hipError_t)error.load();

@@ -16,7 +16,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
-#include <mutex>
 
 namespace vlbm {
 namespace detail {
@@ -26,32 +25,22 @@ struct FieldCopy {
     void* out;            // on the host: n doubles, or n values as they are on the device
 };
 
-// Page-locked staging of one owner (a lattice handle, a batch): at most 4
-// slots of 2 MB, allocated by the first download that needs them and freed
-// with the owner. Downloads of one owner from several threads take turns.
+// Downloads from 16 MB on take slots of a pool that all lattices and batches of
+// the process share: 4 of 2 MB for a device, page-locked by the first download
+// that needs them and kept until the process ends. Page-locking and first touching
+// 8 MB takes up to 3 ms, as long as the download of 16 to 40 MB itself, so slots of
+// a handle's own made the first download of a new lattice up to twice as long.
+// Downloads at once from several threads hold different slots; those beyond 4 are
+// freed at the end of their download.
 class HostCopy {
 public:
-    HostCopy() = default;
-    HostCopy(const HostCopy&) = delete;
-    HostCopy& operator=(const HostCopy&) = delete;
-    ~HostCopy() { release(); }
     // The fields, after everything enqueued on the stream so far; returns when they are in place. As doubles, or
     // raw as they are on the device.
-    hipError_t fetch(int device, hipStream_t stream, const FieldCopy* fields, int count, size_t n, int value_bytes,
-                     bool raw = false);
-    void release();
+    static hipError_t fetch(int device, hipStream_t stream, const FieldCopy* fields, int count, size_t n,
+                            int value_bytes, bool raw = false);
 
 private:
     static hipError_t fetch_small(hipStream_t stream, const FieldCopy* fields, int count, size_t n, int value_bytes, bool raw);
-    static constexpr int kSlots = 4;
-    static constexpr size_t kSlotBytes = size_t(2) << 20;
-    hipError_t reserve(int slots, size_t bytes);
-    std::mutex mu_;
-    void* slot_[kSlots] = {};
-    bool pinned_[kSlots] = {};
-    hipEvent_t event_[kSlots] = {};
-    size_t slot_bytes_ = 0;
-    int slots_ = 0;
 };
 
 // out[k] = in[k] for n values of 4 or 8 bytes.
