@@ -537,6 +537,15 @@ struct GlobalPC {
 #pragma unroll
         for (int k = 0; k < kCoef; k++) c[k] = (T)((const S*)p.src)[(int64_t)k * p.stride + nd.idx];
     }
+    // those that population i of the node at offset (dx, dy, dz) is made of
+    __device__ __forceinline__ void coefs(int i, int dx, int dy, int dz, T* c) const {
+        const S* at = (const S*)p.src + node_at(p, nd, dx, dy, dz);
+        const int cx = kCX[i], cy = kCY[i], cz = kCZ[i];
+        const bool need[kCoef] = {true, cx != 0, cy != 0, cz != 0, cx != 0, cy != 0, cz != 0, cx * cy != 0, cx * cz != 0, cy * cz != 0};
+#pragma unroll
+        for (int k = 0; k < kCoef; k++)
+            if (need[k]) c[k] = (T)at[(int64_t)k * p.stride];
+    }
     // Population i of this node in the idle lattice (its post-collision value
     // of the step before the last); read before the step overwrites it.
     __device__ __forceinline__ T held(int i) const {
@@ -554,8 +563,30 @@ __host__ __device__ constexpr int xpair_slot(int i) {
 // Gather (pull streaming) of the post-stream deviations: g_i(x) = g*_i(x - c_i).
 template <int Q, typename T, class PC>
 __device__ __forceinline__ void gather(T* g, PC pc) {
+    if constexpr (PC::kCoefs && (Q == 27) == (sizeof(T) == 4)) {
+        // The coefficients of the next three populations are loaded before
+        // these three are rebuilt. What bounds these passes is the latency of 90
+        // (D3Q27: 170) loads, and left to itself the compiler waits for each
+        // of them here: 130^2 x 120 walls, us, so and grouped, D3Q27 float 253
+        // 89, D3Q19 double 163 112. The other two it schedules better itself
+        // (D3Q19 float 59, grouped 61; D3Q27 double 215, grouped 325).
+        constexpr int G = 3;
+        T c[2][G][kCoef];
+        auto fetch = [&](int i0, T (*to)[kCoef]) {
 #pragma unroll
-    for (int i = 0; i < Q; i++) g[i] = pc(i, -kCX[i], -kCY[i], -kCZ[i]);
+            for (int i = i0; i < i0 + G && i < Q; i++) pc.coefs(i, -kCX[i], -kCY[i], -kCZ[i], to[i - i0]);
+        };
+        fetch(0, c[0]);
+#pragma unroll
+        for (int i0 = 0; i0 < Q; i0 += G) {
+            fetch(i0 + G, c[(i0 / G + 1) & 1]);
+#pragma unroll
+            for (int i = i0; i < i0 + G && i < Q; i++) g[i] = recon<Q, T, T>(i, c[i0 / G & 1][i - i0], 1);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < Q; i++) g[i] = pc(i, -kCX[i], -kCY[i], -kCZ[i]);
+    }
 }
 
 // Pull streaming of populations with the x shift done in LDS. Each thread of
