@@ -1157,7 +1157,8 @@ template <int Q, typename S, int RHEO, bool MASK, bool DIRECT, bool IBM = false,
           bool ROWS = false>
 __global__ __launch_bounds__(kBlock) void k_step(const Params<typename ComputeOf<S>::type> p) {
     static_assert(!ROWS || (!DIRECT && IN == kRepPop), "the row pull reads populations of the previous step");
-    const uint32_t idx = (ROWS ? blockIdx.x : step_block(p)) * kBlock + threadIdx.x;
+    constexpr bool kStreams = ROWS || DIRECT || sizeof(S) == 2;      // never cached (cached_step)
+    const uint32_t idx = (kStreams ? blockIdx.x : step_block(p)) * kBlock + threadIdx.x;
     if constexpr (ROWS) {
         __shared__ typename ComputeOf<S>::type sm[XShifted<Q>::count() * kBlock];
         const bool in = idx < p.n;                            // the grid holds no block wholly past the lattice

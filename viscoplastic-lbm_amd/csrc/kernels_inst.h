@@ -36,12 +36,24 @@ struct Inst {
 
     // Whether a population step of two lattices of `bytes` in all stores through
     // the caches (256 MB memory-side cache, 8 x 4 MB L2) and runs back and forth,
-    // instead of streaming past them. D3Q19, us a step, streaming and cached:
-    // 30 MB 7.2 7.8, 56 MB 14.4 12.1, 134 MB 28.4 23.9, 237 MB 45.8 40.2,
-    // 398 MB 78.5 74.7, 456 MB 95.0 87.3, 840 MB (double) 158 157. Below, the
-    // write-back at the kernel's end costs more; above, little is left of the
-    // step before. The row pull keeps streaming (80 MB 18.1 19.5, 319 MB 65.1 68.8).
-    static int cached_step(double bytes) { return bytes >= 40e6 && bytes <= 512e6 ? 1 : 0; }
+    // instead of streaming past them. Below the range the write-back at the
+    // kernel's end costs more; above it, little is left of the step before. us a
+    // step, streaming and cached:
+    //   D3Q19 box maps      38 MB 10.2 10.7, 45 MB 12.7 10.2, 90 MB 22.5 17.6, 180 MB 38.6 30.9,
+    //                       320 MB 63.8 61.1, 430 MB 84.0 80.5, 456 MB 95.0 87.3, 540 MB 100 102 (double)
+    //   with the power law  380 MB 73.3 72.4, 438 MB 81.6 83.8, 480 MB 91.2 93.0 (omega's two fields on top)
+    //   D3Q27 float         45 MB 13.3 11.3, 250 MB 52.3 43.6, 320 MB 63.4 63.8, 430 MB 84.7 86.2
+    //   D3Q27 double        45 MB 11.3 12.1, 60 MB 16.2 15.6, 320 MB 64.6 63.6, 480 MB 93.7 92.9
+    //   node maps (D3Q19)   45 MB 16.9 14.7, 250 MB 54.3 48.1, 320 MB 73.6 75.0, 430 MB 88.8 95.9
+    // The row pull keeps streaming (80 MB 18.1 19.5, 319 MB 65.1 68.8), and so does
+    // 16-bit storage, which gains nothing (D3Q19 130 MB 32.1 32.6).
+    template <int Q, int RHEO, bool MASK>
+    static int cached_step(double bytes) {
+        const bool d27 = Q == 27 && sizeof(S) == 8;
+        const double lo = d27 && !MASK ? 50e6 : 40e6;
+        const double hi = MASK || (Q == 27 && !d27) ? 300e6 : (RHEO == 2 ? 400e6 : 480e6);
+        return sizeof(S) > 2 && bytes >= lo && bytes <= hi ? 1 : 0;
+    }
 
     template <int Q, int RHEO, bool MASK, bool IBM>
     static void step_pop(bool direct, const Params<T>& p, hipStream_t st) {
@@ -58,7 +70,7 @@ struct Inst {
             }
         }
         Params<T> pc = p;
-        pc.cached = cached_step(2.0 * Q * sizeof(S) * p.n);
+        pc.cached = cached_step<Q, RHEO, MASK>(2.0 * Q * sizeof(S) * p.n);
         hipLaunchKernelGGL((k_step<Q, S, RHEO, MASK, false, IBM>), grid_of(p.n), dim3(kBlock), 0, st, pc);
     }
 
