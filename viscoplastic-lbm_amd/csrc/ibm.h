@@ -125,4 +125,18 @@ enum IbmStagePart : int {
 // 2 ceil(r) + 6 nodes per axis.
 inline int ibm_box_edge(double r_max) { return 2 * (int)std::ceil(r_max) + 6; }
 
+// k_ibm_spread_box: its threads, the nodes of a batch, and the LDS it holds
+// beside the box (position and force of the batch's nodes, and records of the
+// reduction and of overlapping boxes, 528 bytes).
+constexpr int kSphereBlock = 1024;
+constexpr int kSpreadBatch = 512;
+constexpr size_t kSpreadLds = 6 * sizeof(double) * kSpreadBatch + 1024;
+
+// Edge of the box where a whole one (many spheres take one slab each) fits a
+// workgroup's LDS beside that; else 0. 160 KB hold it for radii up to 8, 125 KB.
+inline int ibm_lds_box_edge(double r_max, size_t lds_bytes) {
+    const size_t edge = (size_t)ibm_box_edge(r_max);
+    return 3 * sizeof(int) * edge * edge * edge + kSpreadLds <= lds_bytes ? (int)edge : 0;
+}
+
 }  // namespace vlbm

@@ -33,13 +33,10 @@ void update_cells(const vlbm_ctx* h, IbmState& s) {
     // LDS spreading box for FP32 fluids when it fits the workgroup's LDS
     s.P.box_edge = 0;
     if (h->tbytes == 4 && s.r_max > 0) {
-        const int edge = ibm_box_edge(s.r_max);
-        const size_t bytes = 3 * sizeof(int) * (size_t)edge * edge * edge;
         hipDeviceProp_t prop;
         int dev = 0;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess &&
-            bytes + 4096 <= prop.sharedMemPerBlock)
-            s.P.box_edge = edge;
+        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
+            s.P.box_edge = ibm_lds_box_edge(s.r_max, prop.sharedMemPerBlock);
     }
     // plain stores into box nodes need every lattice node to appear once in a
     // box: no periodic axis shorter than the box

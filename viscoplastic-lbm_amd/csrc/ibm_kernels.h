@@ -743,7 +743,6 @@ __device__ __forceinline__ bool node_stencil(const IbmParams& P, const double po
 // of 4 neighbouring nodes. Lanes 0..11 evaluate the 12 kernel weights and
 // the others read theirs with shuffles.
 constexpr int kInterpBlock = 256;
-constexpr int kSphereBlock = 1024;
 constexpr int kRowLanesShare = 16;   // lanes per node in the row-parallel kernels
 
 struct PointOf {
@@ -1020,7 +1019,6 @@ __global__ __launch_bounds__(kInterpBlock) void k_ibm_spread(IbmParams P, IbmFlu
 // contribution is at most 2^-31 of the sphere's force sum. A sphere whose
 // force sum is not finite spreads through the global float atomics, so that
 // the fluid sees the same NaN or infinity as the sphere.
-constexpr int kSpreadBatch = 512;     // nodes; 24 KB beside a whole box of at most 128 KB
 __device__ __forceinline__ int box_fixed(double v, double s) { return (int)rint(v * s); }
 
 __global__ __launch_bounds__(kSphereBlock) void k_ibm_spread_box(IbmParams P, IbmFluid<float> fl) {
