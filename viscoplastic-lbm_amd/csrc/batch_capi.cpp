@@ -22,12 +22,12 @@
 #include <deque>
 #include <map>
 #include <memory>
-#include <new>
 #include <string>
 #include <vector>
 
 #include "batch.h"
 #include "ctx.h"
+#include "result_pool.h"
 
 using namespace vlbm;
 using namespace vlbm::detail;
@@ -87,8 +87,7 @@ struct vlbm_batch {
     std::string tuned_key;                     // resident-node bucket the launch shape was chosen for
     bool fixed_shape = false;                  // K, block and grid given by the caller
     std::map<std::string, std::array<int, 3>> shapes;   // launch shapes chosen in this batch, by key
-    std::multimap<size_t, std::unique_ptr<char[]>> spare;   // released result buffers by size
-    size_t spare_bytes = 0;
+    ResultPool results;                        // released result buffers
     int device = 0;                            // device current at vlbm_batch_create (the stream's device)
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -254,34 +253,6 @@ int admit(vlbm_batch* b, int id) {
     return VLBM_OK;
 }
 
-// Result buffers. Released ones are kept for later jobs, at most kSpareBytes of
-// them in a batch: a fresh buffer costs its page faults, as much time as its copy.
-constexpr size_t kSpareBytes = size_t(256) << 20;
-
-int take_result(vlbm_batch* b, Job& j, size_t bytes) {
-    auto best = b->spare.lower_bound(bytes);
-    if (best != b->spare.end() && best->first <= 2 * bytes) {
-        j.res_bytes = best->first;
-        j.res = std::move(best->second);
-        b->spare_bytes -= best->first;
-        b->spare.erase(best);
-        return VLBM_OK;
-    }
-    j.res.reset(new (std::nothrow) char[bytes]);
-    if (!j.res) return fail(VLBM_ERR_ALLOC, "result of a job: host allocation failed");
-    j.res_bytes = bytes;
-    return VLBM_OK;
-}
-
-void give_result(vlbm_batch* b, Job& j) {
-    if (j.res && b->spare_bytes + j.res_bytes <= kSpareBytes) {
-        b->spare_bytes += j.res_bytes;
-        b->spare.emplace(j.res_bytes, std::move(j.res));
-    }
-    j.res.reset();
-    j.res_bytes = 0;
-}
-
 // final macroscopics into the idle lattice of the job, then to the host
 int retire(vlbm_batch* b, int id, int state) {
     Job& j = b->jobs[id];
@@ -308,7 +279,8 @@ int retire(vlbm_batch* b, int id, int state) {
         rc = launch_aux(j.d.q, j.d.precision, j.d.rheology, false, &p, b->stream);
     }
     if (rc) return check_launch(rc, "final moments");
-    if ((rc = take_result(b, j, 4 * fb))) return rc;
+    j.res = b->results.take(4 * fb, &j.res_bytes);
+    if (!j.res) return fail(VLBM_ERR_ALLOC, "result of a job: host allocation failed");
     FieldCopy fields[4];
     for (int f = 0; f < 4; f++) fields[f] = FieldCopy{idle + f * fb, j.res.get() + f * fb};
     HIP_TRY(HostCopy::fetch(b->device, b->stream, fields, 4, n, b->tbytes, true));
@@ -755,8 +727,9 @@ int vlbm_batch_release(vlbm_batch_h b, int job) {
     if (rc) return rc;
     if (job < 0 || job >= (int)b->jobs.size()) return fail(VLBM_ERR_INVALID, "unknown job");
     Job& j = b->jobs[job];
-    give_result(b, j);
+    if (!j.has_result) return VLBM_OK;
     j.has_result = false;
+    b->results.give(std::move(j.res), j.res_bytes);
     return VLBM_OK;
 }
 
