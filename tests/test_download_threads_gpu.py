@@ -71,3 +71,16 @@ def test_callers_at_once():
     assert same == [True] * 4
     for lat, _ in made:
         lat.close()
+
+
+def test_fields_of_a_refused_call():
+    """A Newtonian fluid has no omega: the call fails, with the other fields in place."""
+    import ctypes as C
+    from vlbm._capi import lib
+    lat, want = make((9, 8, 7), "double")
+    out = {k: np.full(lat.shape, np.nan) for k in KEYS + ("omega",)}
+    rc = lib.vlbm_macroscopics(lat._h, *[out[k].ctypes.data_as(C.POINTER(C.c_double)) for k in KEYS + ("omega",)])
+    assert rc != 0 and np.isnan(out["omega"]).all()
+    for k in KEYS:
+        assert np.array_equal(out[k], want[k]), k
+    lat.close()

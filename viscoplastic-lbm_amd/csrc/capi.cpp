@@ -839,10 +839,12 @@ int vlbm_macroscopics(vlbm_h h, double* rho, double* ux, double* uy, double* uz,
     int count = 0;
     for (int k = 0; k < 5; k++) {
         if (!outs[k]) continue;
-        if (!h->macr[k]) return fail(VLBM_ERR_INVALID, "omega exists for non-Newtonian fluids only");
-        fields[count++] = FieldCopy{h->macr[k], outs[k]};
+        if (h->macr[k]) fields[count++] = FieldCopy{h->macr[k], outs[k]};
     }
-    return fetch_fields(h, fields, count);
+    if (int rc = fetch_fields(h, fields, count)) return rc;
+    // the call fails, with the other fields in place
+    if (omega && !h->macr[4]) return fail(VLBM_ERR_INVALID, "omega exists for non-Newtonian fluids only");
+    return VLBM_OK;
 }
 
 int vlbm_visc_turb(vlbm_h h, double* out) {
