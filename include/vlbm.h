@@ -55,8 +55,8 @@ extern "C" {
  * and double storage, regularized collision only): 10 instead of Q values
  * read and written per node. AUTO: MOMENTS in float storage with the
  * regularized collision, for every builder but the rheometer, when NX >= 64
- * and the lattice holds at least 2,048 tiles of 64 x 8 nodes (64 x 4 for
- * D3Q27 and for the duct builders' node maps) by 4 planes; else POPULATIONS.
+ * and the lattice holds at least 2,048 units of 64 x 8 x 4 nodes (64 x 4 x 4 for
+ * D3Q27 and for the duct builders' node maps); else POPULATIONS.
  * vlbm_layout reports the choice. */
 #define VLBM_LAYOUT_AUTO 0
 #define VLBM_LAYOUT_POPULATIONS 1

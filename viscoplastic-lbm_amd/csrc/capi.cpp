@@ -372,14 +372,14 @@ int vlbm_create(const vlbm_desc* d, vlbm_h* out) {
         release(h);
         return fail(VLBM_ERR_DEVICE, "hipEventCreate failed");
     }
-    // AUTO: coefficients in float storage, where they are faster on MI355X
-    // (GLUPS, coefficients vs populations: 256^3 D3Q19 Bingham duct 56.0 vs 38.6;
-    // with the tile kernel's predecessor, 256^3: D3Q19 plates 44.4 vs 39.4,
-    // power-law plates 37.7 vs 37.1, circular duct 32.6 vs 30.8, annular 32.0 vs
-    // 29.1, D3Q27 power-law plates 31.0 vs 24.8, D3Q27 circular duct 29.2 vs
-    // 21.6). FP64 runs faster with populations, and the rheometer's plates hold
-    // populations. Lattices of less than 2,048 tiles (64 x 8 or 64 x 4 nodes, 4
-    // planes) keep populations, one thread per node.
+    // AUTO: coefficients in float storage from 2,048 units of 64 x 8 x 4 nodes on
+    // (64 x 4 x 4 for D3Q27 and node maps; the tiles of the kernel are 64 x 8 there
+    // too). us a step, populations and coefficients, around that line: D3Q19 plates
+    // 128 x 128 x 256 119 93; circular duct 128^3 83 70, 130^3 69 91 (rows that leave
+    // tiles a third empty); D3Q27 plates 128^3 90 52, 130^3 90 76; below it D3Q19
+    // plates 96^3 24 27, 130^3 61 70, but 128^3 65 50. FP64 keeps populations, though
+    // coefficients are faster there where rows fill whole tiles (D3Q19 plates 192^3
+    // 391 286, 130^3 126 133), and the rheometer's plates hold populations.
     const int tile_rows = (d->q == 19 && !h->mask_geom) ? 8 : 4;
     const long tiles = (long)((d->nx + 63) / 64) * ((d->ny + tile_rows - 1) / tile_rows) * ((d->nz + 3) / 4);
     const bool mom_auto = d->collision == VLBM_COLLISION_REGULARIZED && d->precision == VLBM_FP32 && d->nx >= 64 &&

@@ -3,13 +3,15 @@
 // What bounds it is the host: the link carries 55 GB/s, while one thread that
 // lets the runtime stage a pageable copy into a fresh temporary and then
 // converts it writes every page three times and faults it in twice (the four
-// fields of a 256^3 float lattice: 107 ms, of which the link needs 5). From 16 MB
+// fields of a 256^3 float lattice: 96 ms, of which the link needs 5). From 16 MB
 // on, copies go into page-locked slots, all in flight, and are converted from there
 // into place; the destination is faulted in while the stream still computes, which
-// is half of the time. From 128 MB on 4 threads share the chunks: those fields then
-// take 17 ms after an idle stream (8 threads 14, 2 27, 1 45), about 8 behind 200
-// steps. Smaller downloads stay on one thread: with threads a pass of 9 ms and 28 MB
-// took 11.4 or 23 ms, run by run, beside a caller's own spinning pool. Below 16 MB
+// is half of the time (after an idle stream, staging and slots: 16 MB float 4.3 and
+// 2.4 ms, 30 MB 7.7 and 4.7, 125 MB 25 and 19, 17 MB double 1.14 and 0.80). From
+// 128 MB on 4 threads share the chunks: those four fields then take 12 ms (134 MB
+// double 4.8 where staging takes 14). Smaller downloads stay on one thread: with
+// threads a pass of 9 ms and 28 MB took 11.4 or 23 ms, run by run, beside a caller's
+// own spinning pool; between 28 and 125 MB the line was not measured. Below 16 MB
 // the runtime's staging is the faster one (0.6 million float nodes 1.4 ms, slots 1.2
 // to 2.0).
 #pragma once

@@ -32,7 +32,10 @@ template <int Q> struct Moving {
 // bounds test and rows stay conflict-free. Two arrays sets (one barrier per
 // plane) where two workgroups per CU fit 160 KB with them, else one set and
 // two barriers: 75.1 KB float D3Q19, 56.4 KB float D3Q27 (both 64 x 8),
-// 42.1 KB and 62.9 KB double (64 x 4).
+// 42.1 KB and 62.9 KB double (64 x 4). 256^3, us a step with the kernel that
+// rebuilt pulled populations at their receiver and with this one: D3Q19 Bingham
+// duct 397 300, circular duct 514 415 to 421, D3Q27 plates 461 304, double D3Q19
+// plates 160 x 160 x 128 271 163.
 template <typename T, int Q> struct TileShape {
     static constexpr int TY = sizeof(T) == 4 ? 8 : 4;
     static constexpr int NT = kTileX * TY;
@@ -283,6 +286,8 @@ __global__ __launch_bounds__((TileShape<T, Q>::NT), (TileShape<T, Q>::MIN_WAVES)
 
 // z-chunk per workgroup: 32 planes, fewer until the lattice has enough
 // workgroups to fill the device in whole rounds (two per CU: 2,048 are 4 rounds).
+// The number comes from a kernel with another tile loop and was not swept with
+// this one; a chunk reads two planes more than it completes.
 inline int tile_zchunk(int nx, int ny, int nz, int ty) {
     const long tiles = (long)((nx + kTileX - 1) / kTileX) * ((ny + ty - 1) / ty);
     int zc = 32;
