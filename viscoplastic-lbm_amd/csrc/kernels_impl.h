@@ -528,6 +528,7 @@ struct GlobalPC {
     // coefficient states: the node's own 10 coefficients, read once for the
     // several populations a bounce-back rebuilds from them
     static constexpr bool kCoefs = IN == kRepMom;
+    static constexpr bool kFaces = kCoefs || (Q == 19 && sizeof(S) > 2);      // free slip compiled face by face
     static constexpr bool kPlates = IN == kRepPop;      // the rheometer is refused for coefficients
     __device__ __forceinline__ void fence() const {}
     // wall weights of the column (ibb_index)
@@ -770,7 +771,7 @@ __device__ __forceinline__ void apply_bc(T* g, const Params<T>& p, const Node<T>
                 if (m & (1u << i)) g[i] = pc(opp(i), 0, 0, 0);
         }
     } else if (scheme == kFreeSlip) {
-        if constexpr (PC::kCoefs) {
+        if constexpr (PC::kFaces) {
             switch (dir) {
             case dN: free_slip_face<Q, dN>(g, pc); break;
             case dS: free_slip_face<Q, dS>(g, pc); break;
@@ -781,10 +782,11 @@ __device__ __forceinline__ void apply_bc(T* g, const Params<T>& p, const Node<T>
             default: break;
             }
         } else {
-            // populations: one loop for all faces. Compiled face by face it made
-            // D3Q27 steps spill and cost others registers (us a step, by face and
-            // so: D3Q27 float 430 MB 86.9 81.5, double 480 MB 99.0 94.2, D3Q19
-            // bfloat16 320 MB 82.8 76.7)
+            // One loop for all faces: compiled face by face, D3Q27 steps on
+            // populations spill and 16-bit ones lose registers, also where no
+            // face slips (us a step, by face and so: D3Q27 float 430 MB 86.9
+            // 81.5, double 480 MB 99.0 94.2, D3Q19 bfloat16 320 MB 82.8 76.7).
+            // The others gain where faces slip (D3Q19 30^3 float 5.8 6.6).
             if (dir > dB) return;
             const bool fx = dir == dW || dir == dE, fy = dir == dN || dir == dS, fz = dir == dF || dir == dB;
             const unsigned faces = kDirFaces[dir];

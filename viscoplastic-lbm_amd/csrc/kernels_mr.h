@@ -61,7 +61,7 @@ struct ColumnPC {
     GlobalPC<Q, T, T, kRepMom> far;
     __device__ __forceinline__ T operator()(int i, int, int, int) const { return recon<Q, T, T>(i, c, 1); }
     __device__ __forceinline__ T memory(int i, int dx, int dy, int dz) const { return far(i, dx, dy, dz); }
-    static constexpr bool kCoefs = true, kPlates = false;
+    static constexpr bool kCoefs = true, kFaces = true, kPlates = false;
     // wall weights: the same on every plane, so read when the wall changes
     __device__ __forceinline__ void walls(bool inside) const {
         const int w = inside ? 1 : 2;
