@@ -51,6 +51,14 @@ def test_box_map_population_steps_do_not_spill(q):
     assert not {n: s for n, s in step.items() if s}
 
 
+def test_half_precision_row_pull_runs_six_waves():
+    """Box-map D3Q19 steps of 16-bit storage: 512 registers a SIMD lane hold six waves of up to 80."""
+    step = {n: k[".vgpr_count"] for n, k in kernels().items()
+            if re.match(r"_ZN4vlbm6k_stepILi19E(DF16_|NS_4bf16E)Li[012]ELb0ELb0ELb0ELi0ELi0E", n)}
+    assert len(step) == 12
+    assert not {n: v for n, v in step.items() if v > 80}
+
+
 def test_spreading_box_leaves_room_for_the_rest_of_the_kernel(tmp_path):
     (beside,) = [k[".group_segment_fixed_size"] for n, k in kernels().items() if "k_ibm_spread_box" in n]
     (tmp_path / "edges.cpp").write_text("""

@@ -1153,11 +1153,18 @@ __device__ __forceinline__ void step_node_rows(const Params<typename ComputeOf<S
     collide_store<Q, S, RHEO, kRepPop, OUT>(p, idx, g, node_force<IBM>(p, nd), RHEO == 2 ? p.omega_state[idx] : (T)0);
 }
 
+// Waves per SIMD the register allocation of k_step must allow (0: as it comes).
+// The D3Q19 box-map steps of 16-bit storage are at the edge of 6 (80 registers); the
+// half Newtonian row pull took 88 and ran 5 waves: 128 x 128 x 200 73 us a step with
+// 79 registers, 79 with 88.
+template <int Q, typename S, bool MASK, bool DIRECT, bool IBM>
+constexpr int step_waves() { return sizeof(S) == 2 && Q == 19 && !MASK && !DIRECT && !IBM ? 6 : 0; }
+
 // One time step over the lattice, one node per thread; ROWS: pull through
 // gather_rows (populations, not direct).
 template <int Q, typename S, int RHEO, bool MASK, bool DIRECT, bool IBM = false, int IN = kRepPop, int OUT = kRepPop,
           bool ROWS = false>
-__global__ __launch_bounds__(kBlock) void k_step(const Params<typename ComputeOf<S>::type> p) {
+__global__ __launch_bounds__(kBlock, (step_waves<Q, S, MASK, DIRECT, IBM>())) void k_step(const Params<typename ComputeOf<S>::type> p) {
     static_assert(!ROWS || (!DIRECT && IN == kRepPop), "the row pull reads populations of the previous step");
     constexpr bool kStreams = ROWS || DIRECT || sizeof(S) == 2;      // never cached (cached_step)
     const uint32_t idx = (kStreams ? blockIdx.x : step_block(p)) * kBlock + threadIdx.x;
