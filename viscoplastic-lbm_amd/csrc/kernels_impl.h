@@ -618,13 +618,13 @@ template <int Q> struct XShifted {
     }
 };
 
-// Block of nodes a workgroup takes. Cached steps (Params::cached) go back and
+// Block of nodes a workgroup of a cached step takes: the steps go back and
 // forth through the lattice, so that what the step before wrote last is read
 // first. Blocks keep their residue mod 8, the XCD they run on.
 template <typename T>
 __device__ __forceinline__ uint32_t step_block(const Params<T>& p) {
     const uint32_t octets = gridDim.x / 8u, o = blockIdx.x / 8u;
-    if (!p.cached || !p.odd || o >= octets) return blockIdx.x;
+    if (!p.odd || o >= octets) return blockIdx.x;
     return (octets - 1u - o) * 8u + blockIdx.x % 8u;
 }
 
@@ -1032,8 +1032,9 @@ __device__ __forceinline__ Force<T> node_force(const Params<T>& p, const Node<T>
 
 // Moments, apparent omega, saved macroscopics and collision of one node whose
 // post-stream, post-BC deviations are g; the post-collision state goes to
-// dst in representation OUT. om_old: the power law's omega of the node.
-template <int Q, typename S, int RHEO, int IN, int OUT>
+// dst in representation OUT. om_old: the power law's omega of the node. CACHED:
+// populations are stored through the caches instead of past them.
+template <int Q, typename S, int RHEO, int IN, int OUT, bool CACHED = false>
 __device__ __forceinline__ void collide_store(const Params<typename ComputeOf<S>::type>& p, uint32_t idx,
                                               typename ComputeOf<S>::type* g,
                                               const Force<typename ComputeOf<S>::type>& F,
@@ -1070,17 +1071,12 @@ __device__ __forceinline__ void collide_store(const Params<typename ComputeOf<S>
             return;
         }
     }
-    if (sizeof(S) > 2 && p.cached) {
-        // the empty asm keeps the compiler from merging the two branches into
-        // one set of stores, which drops the non-temporal hint
-        asm volatile("");
 #pragma unroll
-        for (int i = 0; i < Q; i++) st<S, T>(dst + (int64_t)i * p.stride + idx, g[i]);
-        asm volatile("");
-        return;
+    for (int i = 0; i < Q; i++) {
+        S* at = dst + (int64_t)i * p.stride + idx;
+        if (CACHED) st<S, T>(at, g[i]);
+        else st_nt<S, T>(at, g[i]);
     }
-#pragma unroll
-    for (int i = 0; i < Q; i++) st_nt<S, T>(dst + (int64_t)i * p.stride + idx, g[i]);
 }
 
 // One node of one time step. DIRECT: the source holds the post-stream state
@@ -1088,7 +1084,8 @@ __device__ __forceinline__ void collide_store(const Params<typename ComputeOf<S>
 // IBM: the force of nodes in flagged tiles comes from the IBM force field
 // (src/CUDA/lbm.cu:45-58 reads macr.f per node in IBM builds). IN / OUT:
 // representation of the source and destination lattices.
-template <int Q, typename S, int RHEO, bool MASK, bool DIRECT, bool IBM, int IN = kRepPop, int OUT = kRepPop>
+template <int Q, typename S, int RHEO, bool MASK, bool DIRECT, bool IBM, int IN = kRepPop, int OUT = kRepPop,
+          bool CACHED = false>
 __device__ __forceinline__ void step_node(const Params<typename ComputeOf<S>::type>& p, uint32_t idx) {
     using T = typename ComputeOf<S>::type;
     const Node<T> nd = make_node(p, idx);
@@ -1102,7 +1099,7 @@ __device__ __forceinline__ void step_node(const Params<typename ComputeOf<S>::ty
         gather<Q, T>(g, pc);
         if (w_scheme(word) != kNull) apply_bc<Q, T, MASK>(g, p, nd, word, pc);
     }
-    collide_store<Q, S, RHEO, IN, OUT>(p, idx, g, node_force<IBM>(p, nd), RHEO == 2 ? p.omega_state[idx] : (T)0);
+    collide_store<Q, S, RHEO, IN, OUT, CACHED>(p, idx, g, node_force<IBM>(p, nd), RHEO == 2 ? p.omega_state[idx] : (T)0);
 }
 
 // One pulled step of a population node (gather_rows); every thread of the
@@ -1155,26 +1152,28 @@ __device__ __forceinline__ void step_node_rows(const Params<typename ComputeOf<S
 
 // Waves per SIMD the register allocation of k_step must allow (0: as it comes).
 // The D3Q19 box-map steps of 16-bit storage are at the edge of 6 (80 registers); the
-// half Newtonian row pull took 88 and ran 5 waves: 128 x 128 x 200 73 us a step with
-// 79 registers, 79 with 88.
+// half Newtonian row pull took 88 and ran 5 waves: 128 x 128 x 200 79.1 us a step,
+// 69.4 with the 71 it takes under this bound.
 template <int Q, typename S, bool MASK, bool DIRECT, bool IBM>
 constexpr int step_waves() { return sizeof(S) == 2 && Q == 19 && !MASK && !DIRECT && !IBM ? 6 : 0; }
 
 // One time step over the lattice, one node per thread; ROWS: pull through
-// gather_rows (populations, not direct).
+// gather_rows (populations, not direct). CACHED: stores through the caches, back
+// and forth through the lattice (populations, not direct). A kernel of its own,
+// as a test of a parameter in one kernel cost lattices below the range of
+// cached_step 2 % (D3Q19 float 60 x 66 x 66 10.7 us a step, 11.0 with the test).
 template <int Q, typename S, int RHEO, bool MASK, bool DIRECT, bool IBM = false, int IN = kRepPop, int OUT = kRepPop,
-          bool ROWS = false>
+          bool ROWS = false, bool CACHED = false>
 __global__ __launch_bounds__(kBlock, (step_waves<Q, S, MASK, DIRECT, IBM>())) void k_step(const Params<typename ComputeOf<S>::type> p) {
     static_assert(!ROWS || (!DIRECT && IN == kRepPop), "the row pull reads populations of the previous step");
-    constexpr bool kStreams = ROWS || DIRECT || sizeof(S) == 2;      // never cached (cached_step)
-    const uint32_t idx = (kStreams ? blockIdx.x : step_block(p)) * kBlock + threadIdx.x;
+    const uint32_t idx = (CACHED ? step_block(p) : blockIdx.x) * kBlock + threadIdx.x;
     if constexpr (ROWS) {
         __shared__ typename ComputeOf<S>::type sm[XShifted<Q>::count() * kBlock];
         const bool in = idx < p.n;                            // the grid holds no block wholly past the lattice
         step_node_rows<Q, S, RHEO, MASK, IBM, OUT>(p, in ? idx : p.n - 1, in, sm);
     } else {
         if (idx >= p.n) return;
-        step_node<Q, S, RHEO, MASK, DIRECT, IBM, IN, OUT>(p, idx);
+        step_node<Q, S, RHEO, MASK, DIRECT, IBM, IN, OUT, CACHED>(p, idx);
     }
 }
 

@@ -41,18 +41,18 @@ struct Inst {
     // step, streaming and cached:
     //   D3Q19 box maps      38 MB 10.2 10.7, 45 MB 12.7 10.2, 90 MB 22.5 17.6, 180 MB 38.6 30.9,
     //                       320 MB 63.8 61.1, 430 MB 84.0 80.5, 456 MB 95.0 87.3, 540 MB 100 102 (double)
-    //   with the power law  380 MB 73.3 72.4, 438 MB 81.6 83.8, 480 MB 91.2 93.0 (omega's two fields on top)
+    //   with the power law  380 MB 73.3 72.4, 430 MB 87.0 84.0, 438 MB 81.6 83.8, 480 MB 91.2 93.0
     //   D3Q27 float         45 MB 13.3 11.3, 250 MB 52.3 43.6, 320 MB 63.4 63.8, 430 MB 84.7 86.2
     //   D3Q27 double        45 MB 11.3 12.1, 60 MB 16.2 15.6, 320 MB 64.6 63.6, 480 MB 93.7 92.9
     //   node maps (D3Q19)   45 MB 16.9 14.7, 250 MB 54.3 48.1, 320 MB 73.6 75.0, 430 MB 88.8 95.9
     // The row pull keeps streaming (80 MB 18.1 19.5, 319 MB 65.1 68.8), and so does
     // 16-bit storage, which gains nothing (D3Q19 130 MB 32.1 32.6).
     template <int Q, int RHEO, bool MASK>
-    static int cached_step(double bytes) {
+    static bool cached_step(double bytes) {
         const bool d27 = Q == 27 && sizeof(S) == 8;
         const double lo = d27 && !MASK ? 50e6 : 40e6;
-        const double hi = MASK || (Q == 27 && !d27) ? 300e6 : (RHEO == 2 ? 400e6 : 480e6);
-        return sizeof(S) > 2 && bytes >= lo && bytes <= hi ? 1 : 0;
+        const double hi = MASK || (Q == 27 && !d27) ? 300e6 : (RHEO == 2 ? 435e6 : 480e6);
+        return bytes >= lo && bytes <= hi;
     }
 
     template <int Q, int RHEO, bool MASK, bool IBM>
@@ -69,9 +69,14 @@ struct Inst {
                 return;
             }
         }
-        Params<T> pc = p;
-        pc.cached = cached_step<Q, RHEO, MASK>(2.0 * Q * sizeof(S) * p.n);
-        hipLaunchKernelGGL((k_step<Q, S, RHEO, MASK, false, IBM>), grid_of(p.n), dim3(kBlock), 0, st, pc);
+        if constexpr (sizeof(S) > 2) {
+            if (cached_step<Q, RHEO, MASK>(2.0 * Q * sizeof(S) * p.n)) {
+                hipLaunchKernelGGL((k_step<Q, S, RHEO, MASK, false, IBM, kRepPop, kRepPop, false, true>), grid_of(p.n),
+                                   dim3(kBlock), 0, st, p);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_step<Q, S, RHEO, MASK, false, IBM>), grid_of(p.n), dim3(kBlock), 0, st, p);
     }
 
     template <int Q, int RHEO>
