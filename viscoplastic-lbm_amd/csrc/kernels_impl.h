@@ -514,8 +514,9 @@ __device__ __forceinline__ uint32_t node_at(const Params<T>& p, const Node<T>& n
 }
 
 // Post-collision population i of the node at offset (dx, dy, dz), read from
-// the source lattice in global memory.
-template <int Q, typename S, typename T, int IN>
+// the source lattice in global memory. FORMS: coefficient passes take the boundary
+// conditions in the tile step's forms; without, in loops, and the gather in groups.
+template <int Q, typename S, typename T, int IN, bool FORMS = true>
 struct GlobalPC {
     const Params<T>& p;
     Node<T> nd;
@@ -528,7 +529,8 @@ struct GlobalPC {
     // coefficient states: the node's own 10 coefficients, read once for the
     // several populations a bounce-back rebuilds from them
     static constexpr bool kCoefs = IN == kRepMom;
-    static constexpr bool kFaces = kCoefs || (Q == 19 && sizeof(S) > 2);      // free slip compiled face by face
+    static constexpr bool kFaces = kCoefs ? FORMS : Q == 19 && sizeof(S) > 2;      // free slip compiled face by face
+    static constexpr bool kGroups = kCoefs && ((Q == 27) == (sizeof(T) == 4) || !FORMS);
     static constexpr bool kPlates = IN == kRepPop;      // the rheometer is refused for coefficients
     __device__ __forceinline__ void fence() const {}
     // wall weights of the column (ibb_index)
@@ -564,7 +566,7 @@ __host__ __device__ constexpr int xpair_slot(int i) {
 // Gather (pull streaming) of the post-stream deviations: g_i(x) = g*_i(x - c_i).
 template <int Q, typename T, class PC>
 __device__ __forceinline__ void gather(T* g, PC pc) {
-    if constexpr (PC::kCoefs && (Q == 27) == (sizeof(T) == 4)) {
+    if constexpr (PC::kGroups) {
         // The coefficients of the next three populations are loaded before
         // these three are rebuilt. What bounds these passes is the latency of 90
         // (D3Q27: 170) loads, and left to itself the compiler waits for each
@@ -761,7 +763,7 @@ __device__ __forceinline__ void apply_bc(T* g, const Params<T>& p, const Node<T>
         if (dir >= dNW && w_geom(word)) return;
         if (dir > dSEB) return;
         const uint32_t m = (Q == 19) ? c_bb19.m[dir] : c_bb27.m[dir];
-        if constexpr (PC::kCoefs) {
+        if constexpr (PC::kCoefs && PC::kFaces) {
             T c[kCoef];
             pc.own(c);
             bounce_back<Q, T>(g, c, m);
@@ -1275,7 +1277,9 @@ __global__ __launch_bounds__(kBlock) void k_ibm_macr(const Params<typename Compu
         const uint32_t idx = ((uint32_t)z * (uint32_t)p.ny + (uint32_t)y) * (uint32_t)p.nx + (uint32_t)x;
         const Node<T> nd = make_node(p, idx);
         const uint32_t word = node_word<MASK>(p, nd);
-        const GlobalPC<Q, S, T, IN> pc{p, nd};
+        // D3Q27 double coefficients: the tile step's forms take all 256 registers
+        // (stage of 27 spheres 208 to 216 us, 198 to 200 in loops)
+        const GlobalPC<Q, S, T, IN, !(IN == kRepMom && Q == 27 && sizeof(T) == 8)> pc{p, nd};
         T g[Q];
         if (p.direct || !w_used(word)) {
             load_direct<Q, T>(g, pc);
